@@ -495,13 +495,15 @@ int sq_log_softmax_at(const float* d_logits, size_t n, uint32_t idx, double* out
     if (n == 0) return set_error(SQ_ERR_EMPTY, "log_softmax_at: EmptyInput");
     if (idx >= n) return set_error(SQ_ERR_ARG, "log_softmax_at: index out of range");
     if (n > (size_t)INT32_MAX) return set_error(SQ_ERR_SHAPE, "log_softmax_at: row too long");
-    Tmp id, val, err;
+    Tmp id, val, err, ws;
     int st;
-    if ((st = id.alloc(4)) || (st = val.alloc(8)) || (st = err.alloc(4))) return st;
+    if ((st = id.alloc(4)) || (st = val.alloc(8)) || (st = err.alloc(4)) ||
+        (st = ws.alloc(log_softmax_parts((int)n) * kLsmPartBytes)))
+        return st;
     SQ_HIP_CHECK(hipMemcpy(id.p, &idx, 4, hipMemcpyHostToDevice));
     SQ_HIP_CHECK(hipMemsetAsync(err.p, 0, 4, nullptr));
-    if ((st = launch_log_softmax_at(nullptr, d_logits, (int)n, (const uint32_t*)id.p, (double*)val.p,
-                                    (uint32_t*)err.p)))
+    if ((st = launch_log_softmax_rows(nullptr, d_logits, n, 1, (int)n, (const uint32_t*)id.p, (double*)val.p,
+                                      (uint32_t*)err.p, ws.p)))
         return st;
     if ((st = finish(0))) return st;
     SQ_HIP_CHECK(hipMemcpy(out, val.p, 8, hipMemcpyDeviceToHost));

@@ -464,35 +464,73 @@ __global__ __launch_bounds__(1024) void argmax_final_kernel(const float* logits,
 // log p(idx) under softmax(logits), in f64 (src/bin/perplexity.rs:112-117):
 // the maximum folded in f32 with NaN entries skipped (f32::max), the sum of
 // exp(f64(l) - max) in f64, then f64(l[idx]) - max - ln(sum).  The sum is a
-// fixed-order tree over the workgroup, not the reference's sequential fold,
-// so the two agree to f64 rounding.
-__global__ __launch_bounds__(1024) void log_softmax_at_kernel(const float* __restrict__ logits, int n,
-                                                              const uint32_t* __restrict__ idx,
-                                                              double* __restrict__ out,
-                                                              uint32_t* __restrict__ id_error) {
-    __shared__ float s_m[16];
-    __shared__ double s_s[16];
+// fixed-order tree, not the reference's sequential fold, so the two agree to
+// f64 rounding.
+//
+// One workgroup over a 128256-entry row was bound by its f64 exponentials on
+// one CU (69 us); here a row's chunks of kLsmChunk entries go to a workgroup
+// each, and a wavefront per row then rebases the chunks' sums to the row's
+// maximum.  Several rows share one launch (grid y).
+struct LsmPart {
+    double s;  // sum over the chunk of exp(l - m)
+    float m;   // the chunk's maximum, NaN entries skipped
+    float pad;
+};
+static_assert(sizeof(LsmPart) == kLsmPartBytes, "the workspace holds kLsmPartBytes a chunk");
+
+__global__ __launch_bounds__(kBlock) void log_softmax_parts_kernel(const float* __restrict__ logits, size_t stride,
+                                                                   int n, int chunk, LsmPart* __restrict__ parts) {
+    __shared__ float s_m[kBlock / 64];
+    __shared__ double s_s[kBlock / 64];
     const int tid = threadIdx.x;
+    const float* row = logits + blockIdx.y * stride;
+    const int b0 = min((int64_t)n, (int64_t)blockIdx.x * chunk), b1 = min((int64_t)n, (int64_t)b0 + chunk);
     float m = -INFINITY;
-    for (int i = tid; i < n; i += 1024) m = fmaxf(m, logits[i]);
+    for (int i = b0 + tid; i < b1; i += kBlock) m = fmaxf(m, row[i]);
     m = sq_wave_max(m);
     if ((tid & 63) == 0) s_m[tid >> 6] = m;
     __syncthreads();
     float mx = -INFINITY;
-    for (int w = 0; w < 16; w++) mx = fmaxf(mx, s_m[w]);
+    for (int w = 0; w < kBlock / 64; w++) mx = fmaxf(mx, s_m[w]);
+    // entries of -inf add nothing, also where the chunk has no others (there
+    // exp(l - max) would be NaN); NaN entries poison the sum
     const double md = (double)mx;
     double s = 0.0;
-    for (int i = tid; i < n; i += 1024) s += exp((double)logits[i] - md);
+    for (int i = b0 + tid; i < b1; i += kBlock) {
+        const float l = row[i];
+        if (l != -INFINITY) s += exp((double)l - md);
+    }
     for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
     if ((tid & 63) == 0) s_s[tid >> 6] = s;
     __syncthreads();
     if (tid == 0) {
         double tot = 0.0;
-        for (int w = 0; w < 16; w++) tot += s_s[w];
+        for (int w = 0; w < kBlock / 64; w++) tot += s_s[w];
+        parts[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = LsmPart{tot, mx, 0.0f};
+    }
+}
+
+// out[r] for row r = blockIdx.x from its n_parts chunks.
+__global__ __launch_bounds__(64) void log_softmax_final_kernel(const float* __restrict__ logits, size_t stride, int n,
+                                                               const LsmPart* __restrict__ parts, int n_parts,
+                                                               const uint32_t* __restrict__ idx,
+                                                               double* __restrict__ out,
+                                                               uint32_t* __restrict__ id_error) {
+    const int r = blockIdx.x, lane = threadIdx.x;
+    const LsmPart* p = parts + (size_t)r * n_parts;
+    float mx = -INFINITY;
+    for (int k = lane; k < n_parts; k += 64) mx = fmaxf(mx, p[k].m);
+    mx = sq_wave_max(mx);
+    const double md = (double)mx;
+    // (a row of -inf alone: exp(-inf + inf) is NaN, the reference's result)
+    double s = 0.0;
+    for (int k = lane; k < n_parts; k += 64) s += p[k].s * exp((double)p[k].m - md);
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0) {
         // an index past the row is the reference's panic (perplexity.rs:112-117)
-        const uint32_t i = *idx;
+        const uint32_t i = idx[r];
         if (i >= (uint32_t)n) *id_error = 1u;
-        *out = i < (uint32_t)n ? (double)logits[i] - md - log(tot) : (double)NAN;
+        out[r] = i < (uint32_t)n ? (double)logits[r * stride + i] - md - log(s) : (double)NAN;
     }
 }
 
@@ -631,11 +669,18 @@ int launch_block_isums(hipStream_t s, const int8_t* aq, const MatView& w, int wt
     return check_launch("block_isums");
 }
 
-int launch_log_softmax_at(hipStream_t s, const float* logits, int n, const uint32_t* idx, double* out,
-                          uint32_t* id_error) {
-    if (!id_error) return set_error(SQ_ERR_ARG, "log_softmax_at: no error word");
-    hipLaunchKernelGGL(log_softmax_at_kernel, dim3(1), dim3(1024), 0, s, logits, n, idx, out, id_error);
-    return check_launch("log_softmax_at");
+int launch_log_softmax_rows(hipStream_t s, const float* logits, size_t stride, int rows, int n, const uint32_t* idx,
+                            double* out, uint32_t* id_error, void* ws) {
+    if (!id_error) return set_error(SQ_ERR_ARG, "log_softmax: no error word");
+    if (rows <= 0) return 0;
+    const int parts = log_softmax_parts(n);
+    const int chunk = (int)(((int64_t)n + parts - 1) / parts);
+    hipLaunchKernelGGL(log_softmax_parts_kernel, dim3(parts, rows), dim3(kBlock), 0, s, logits, stride, n, chunk,
+                       (LsmPart*)ws);
+    if (const int st = check_launch("log_softmax")) return st;
+    hipLaunchKernelGGL(log_softmax_final_kernel, dim3(rows), dim3(64), 0, s, logits, stride, n, (const LsmPart*)ws,
+                       parts, idx, out, id_error);
+    return check_launch("log_softmax");
 }
 
 int launch_copy_i32(hipStream_t s, const int* src, int* dst) {

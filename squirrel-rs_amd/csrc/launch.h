@@ -126,9 +126,18 @@ int launch_argmax_partials(hipStream_t s, const float* logits, int n, float* par
 int launch_block_isums(hipStream_t s, const int8_t* aq, const MatView& w, int wtype, int row,
                        int32_t* out);
 int launch_copy_i32(hipStream_t s, const int* src, int* dst);
-// out = log p(*idx) under softmax(logits[0..n)) in f64 (*idx < n).
-int launch_log_softmax_at(hipStream_t s, const float* logits, int n, const uint32_t* idx, double* out,
-                          uint32_t* id_error);
+// out[r] = log p(idx[r]) under softmax(row r) in f64, for `rows` rows of n
+// logits, `stride` floats apart (idx[r] < n, else *id_error is raised).  ws:
+// rows * log_softmax_parts(n) * kLsmPartBytes bytes.
+constexpr int kLsmChunk = 2048;    // logits per workgroup (8 per thread) ...
+constexpr int kLsmMaxParts = 512;  // ... up to this many workgroups a row
+constexpr size_t kLsmPartBytes = 16;
+inline int log_softmax_parts(int n) {
+    const int64_t p = ((int64_t)n + kLsmChunk - 1) / kLsmChunk;
+    return (int)(p < 1 ? 1 : p > kLsmMaxParts ? kLsmMaxParts : p);
+}
+int launch_log_softmax_rows(hipStream_t s, const float* logits, size_t stride, int rows, int n, const uint32_t* idx,
+                            double* out, uint32_t* id_error, void* ws);
 
 // ---- prefill matmul (k_gemm.hip) ----------------------------------------
 // out[m, rows] (+)= in[m, k] @ W.  a8: activations given as Q8_0 (aq/ad,

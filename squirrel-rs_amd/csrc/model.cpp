@@ -883,8 +883,9 @@ int ctx_create(const sq_model* m, size_t max_pos, uint32_t flags, sq_ctx** out) 
         (st = dmalloc(&c->pv, c->n_parts)) ||
         (st = dmalloc(&c->pi, c->n_parts)) || (st = dmalloc(&c->pn, c->n_parts)) ||
         (st = dmalloc(&c->dbg_normed, D)) || (st = dmalloc(&c->last_hidden, D)) || (st = dmalloc(&c->head_qs, D)) ||
-        (st = dmalloc(&c->head_d, D / 32)) || (st = dmalloc(&c->d_sids, max_pos + 1)) ||
-        (st = dmalloc(&c->d_logp, max_pos + 1)) || (st = dmalloc(&c->d_id_error, 1)))
+        (st = dmalloc(&c->head_d, D / 32)) || (st = dmalloc(&c->d_sids, 2 * (max_pos + 1))) ||
+        (st = dmalloc(&c->d_logp, max_pos + 1)) ||
+        (st = dmalloc((uint8_t**)&c->lsm_ws, kScoreRows * (size_t)log_softmax_parts(g.vocab) * kLsmPartBytes)) || (st = dmalloc(&c->d_id_error, 1)))
         return fail(st);
     he = hipHostMalloc((void**)&c->h_pinned, (max_pos + 16) * sizeof(uint32_t), hipHostMallocDefault);
     if (he != hipSuccess) return fail(set_error(SQ_ERR_HIP, std::string("hipHostMalloc: ") + hipGetErrorString(he)));
@@ -943,7 +944,7 @@ void ctx_destroy(sq_ctx* c) {
     dfree(c->p_hidden); dfree(c->p_normed); dfree(c->p_qkv); dfree(c->p_q); dfree(c->p_attn); dfree(c->p_gu);
     dfree(c->p_kvs); dfree(c->p_act); dfree(c->p_aq); dfree(c->p_ad); dfree(c->p_split);
     dfree(c->d_layers); dfree(c->s_stream); dfree(c->s_xchg); dfree(c->s_epoch); dfree(c->s_error); dfree(c->s_trace);
-    dfree(c->d_sids); dfree(c->d_logp); dfree(c->d_id_error);
+    dfree(c->d_sids); dfree(c->d_logp); dfree(c->s_rows); dfree(c->lsm_ws); dfree(c->d_id_error);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -994,17 +995,51 @@ int ctx_score(sq_ctx* c, const uint32_t* ids, size_t n, size_t burn, double* log
     // ctx_forward synchronized before staging the burn-in ids; the window
     // goes to the device behind the prefill on the same stream.
     SQ_HIP_CHECK(hipMemcpyAsync(c->d_sids, ids, n * 4, hipMemcpyHostToDevice, c->stream));
-    // Every step stays on the device: the scored token's log-probability is
-    // taken from the logits in place, and the same id is fed to the next
-    // decode step from device memory.
-    for (size_t i = burn; i < n; i++) {
-        if ((st = launch_log_softmax_at(c->stream, c->logits, V, c->d_sids + i, c->d_logp + (i - burn),
-                                        c->d_id_error)))
-            return st;
-        if (i + 1 < n) {
+    auto log_probs = [&](const float* rows, size_t count, size_t i) {  // of tokens i .. i + count - 1
+        return launch_log_softmax_rows(c->stream, rows, (size_t)V, (int)count, V, c->d_sids + i, c->d_logp + (i - burn),
+                                       c->d_id_error, c->lsm_ws);
+    };
+    if ((st = log_probs(c->logits, 1, burn))) return st;
+    if (c->persist && !c->s_rows && dmalloc(&c->s_rows, (size_t)kScoreRows * V)) {
+        (void)hipGetLastError();  // no room: every step's row is scored in place
+        c->s_rows = nullptr;
+    }
+    if (c->persist && c->s_rows) {
+        // Every step stays on the device, and the persistent steps run back
+        // to back: step i takes its token from a second copy of the window
+        // (it writes the token it would have chosen back there) and writes its
+        // logits to a row of s_rows, and one launch scores kScoreRows rows.  A
+        // log-softmax and a token copy between two steps had taken 74 of 588
+        // us per token.  The last step writes the context's own logits and
+        // token, which stay readable as after any forward.
+        uint32_t* const feed = c->d_sids + (c->max_pos + 1);
+        SQ_HIP_CHECK(hipMemcpyAsync(feed, ids, n * 4, hipMemcpyHostToDevice, c->stream));
+        size_t held = 0;  // rows of s_rows not scored yet: tokens i + 1 - held .. i
+        for (size_t i = burn; i + 1 < n; i++) {
+            StepArgs a = c->step;
+            a.token = feed + i;
+            const bool last = i + 2 == n;
+            if (last) {
+                if ((st = launch_copy_i32(c->stream, (const int*)(feed + i), (int*)c->d_token))) return st;
+                a.token = c->d_token;
+            } else {
+                a.logits = c->s_rows + held * V;
+            }
+            if ((st = launch_decode_step(c->stream, c->m->wtype, a, c->step_grid, (int)c->seq_len))) return st;
+            c->seq_len++;
+            if (!last) held++;
+            if (held == (size_t)kScoreRows || (last && held)) {
+                if ((st = log_probs(c->s_rows, held, (last ? i : i + 1) + 1 - held))) return st;
+                held = 0;
+            }
+            if (last && (st = log_probs(c->logits, 1, i + 1))) return st;
+        }
+    } else {
+        for (size_t i = burn; i + 1 < n; i++) {
             if ((st = launch_copy_i32(c->stream, (const int*)(c->d_sids + i), (int*)c->d_token))) return st;
             if ((st = run_decode_step(c))) return st;
             c->seq_len++;
+            if ((st = log_probs(c->logits, 1, i + 1))) return st;
         }
     }
     SQ_HIP_CHECK(hipMemcpyAsync(logp, c->d_logp, (n - burn) * sizeof(double), hipMemcpyDeviceToHost, c->stream));

@@ -135,8 +135,10 @@ struct sq_ctx {
     // reference's slice index panics there, embedding.rs:43-44); the read
     // itself is clamped in bounds.  Checked by ctx_check, cleared by reset.
     uint32_t* d_id_error = nullptr;
-    uint32_t* d_sids = nullptr;    // the window being scored [max_pos + 1]
+    uint32_t* d_sids = nullptr;    // the window being scored [max_pos + 1], twice (see ctx_score)
     double* d_logp = nullptr;      // its log-probabilities [max_pos + 1]
+    float* s_rows = nullptr;       // logits of scored steps [kScoreRows][vocab], made by the first score
+    void* lsm_ws = nullptr;        // log-softmax partials of kScoreRows rows
     uint32_t* h_pinned = nullptr;  // pinned staging for ids / tokens
     hipGraphExec_t graph = nullptr;
     hipGraph_t graph_def = nullptr;
@@ -176,6 +178,9 @@ int ctx_generate(sq_ctx* c, const uint32_t* prompt, size_t n_prompt, size_t max_
                  uint32_t* out, size_t* n_out, double* step_ms);
 int ctx_time_kernel(sq_ctx* c, int which, int iters, double* mean_us, uint64_t* bytes);
 int ctx_set_taps(sq_ctx* c, bool on);
+// Scored steps whose logits are kept for one log-softmax launch (8.2 MB at a
+// vocabulary of 128256).
+constexpr int kScoreRows = 16;
 // Teacher-forced scoring of one window on a reset context (perplexity.rs:61-110):
 // prefill ids[0, burn), then for i in [burn, n): logp[i - burn] = log p(ids[i])
 // and, while i + 1 < n, one decode step on ids[i].

@@ -504,6 +504,30 @@ def test_score_window_matches_teacher_forced_forward(ppl_gguf, decode):
     assert np.array_equal(c.score(window, burn), got)
 
 
+@pytest.mark.parametrize("steps", [1, 15, 16, 17, 32, 35])
+def test_score_rows_at_batch_edges(ppl_gguf, steps):
+    """Scored steps' logits are kept and scored 16 rows per launch: windows
+    that end before, at and after a full batch give the log-probabilities of
+    the forward loop, and the context's own logits and token are those of the
+    last step."""
+    m = sq.Llama3_2(ppl_gguf)
+    burn = 5
+    window = np.random.default_rng(steps).integers(3, m.vocab, burn + steps + 1).astype(np.uint32)
+    c = m.new_context(64)
+    got = c.score(window, burn)
+    f = m.new_context(64)
+    want = []
+    for i, ids in enumerate([window[:burn]] + [window[k:k + 1] for k in range(burn, window.size - 1)]):
+        f.forward(ids)
+        want.append(seq_log_softmax_at(f.logits(), int(window[burn + i])))
+    assert np.abs(got - np.array(want)).max() < 1e-12
+    assert np.array_equal(c.logits(), f.logits()) and c.argmax() == f.argmax()
+    # decoding goes on from the scored window
+    c.forward([7])
+    f.forward([7])
+    assert np.array_equal(c.logits(), f.logits())
+
+
 def test_perplexity_harness(ppl_gguf):
     """sqhip.perplexity over a token stream: windows of BOS + n_ctx - 1
     tokens, burn-in n_ctx / 2, NLL accumulated in the reference's order;

@@ -551,6 +551,26 @@ def test_log_softmax_at_closed_forms():
         ls(x, 128256)
 
 
+@pytest.mark.parametrize("n", [1, 255, 2047, 2048, 2049, 4097, 512 * 2048 + 5])
+def test_log_softmax_at_chunk_edges(n):
+    """Rows of one partial chunk, whole chunks and chunks longer than the
+    workgroup's; a first chunk that is -inf throughout adds nothing."""
+    x = (rng(n).standard_normal(n) * 4).astype(np.float32)
+    x[:min(n - 1, 2048)] = -np.inf
+    mx = np.float64(x.max())
+    lse = np.log(np.exp(x.astype(np.float64) - mx).sum())
+    d = DeviceArray.from_numpy(x)
+    for i in {n - 1, max(0, n - 2), n // 2}:
+        want = np.float64(x[i]) - mx - lse
+        got = ops.log_softmax_at(d, i)
+        # f64 sums of at most 2^20 terms
+        assert got == want or abs(got - want) < 1e-11
+    if n > 4096:
+        x[n - 3] = np.inf
+        assert np.isnan(ops.log_softmax_at(DeviceArray.from_numpy(x), 0))
+    assert np.isnan(ops.log_softmax_at(DeviceArray.from_numpy(np.full(n, -np.inf, np.float32)), 0))
+
+
 @pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0, O.BF16])
 def test_embed_bit_exact(wtype):
     if wtype == O.BF16:
