@@ -207,6 +207,28 @@ constexpr int MQ_LD = MQ_KC + 8;   // LDS row stride in bytes
 
 typedef int mq_v4i __attribute__((ext_vector_type(4)));
 typedef float sq_v4f __attribute__((ext_vector_type(4)));
+typedef int m8_v16i __attribute__((ext_vector_type(16)));
+typedef float m8_v16f __attribute__((ext_vector_type(16)));
+
+// The block sums reach f32 without a conversion instruction: the integer
+// products accumulate onto kIsumBase, the bit pattern of 1.5 * 2^23, so a
+// result's bits read as the f32 1.5 * 2^23 + isum (exact for |isum| < 2^22;
+// a block's sum is at most 32 * 127 * 128), and one subtraction leaves
+// f32(isum), exactly.  v_cvt_f32_i32 issues at half the rate of a subtraction
+// (2.4 against 1.3 ns per wavefront instruction and SIMD), and with it a
+// 32 x 32 tile and block took 61 ns per SIMD in registers alone, against 41 ns.
+// The base operand sits in registers, behind an empty asm so that the compiler
+// does not set it anew for every product.
+constexpr int kIsumBase = 0x4B400000;
+__device__ __forceinline__ float isum_f32(int d) { return __builtin_bit_cast(float, d) - 12582912.0f; }
+template <typename V>
+__device__ __forceinline__ V isum_base() {
+    V v;
+#pragma unroll
+    for (int r = 0; r < (int)(sizeof(V) / 4); r++) v[r] = kIsumBase;
+    asm volatile("" : "+v"(v));
+    return v;
+}
 typedef _Float16 mq_v4h __attribute__((ext_vector_type(4)));
 
 template <int WT>
@@ -306,6 +328,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(MatView w, const int8_t*
         *(uint2*)&sSw[b][r][0] = (b < 2) ? make_uint2(sw, 0u) : make_uint2(0u, sw);
     };
 
+    const mq_v4i ibase = isum_base<mq_v4i>();
     if (tid < MQ_KB) sSa[MQ_T][tid] = 0;
     fetch(kb_begin);
     for (int kb0 = kb_begin; kb0 < kb_end; kb0 += MQ_KB) {
@@ -333,14 +356,13 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(MatView w, const int8_t*
                 sw[j] = *(const mq_v4h*)&sSw[b][wn + 16 * j + fr][0];
             }
         };
-        const mq_v4i zero = {0, 0, 0, 0};
         const sq_v4f fzero = {0.0f, 0.0f, 0.0f, 0.0f};
         mq_v4i d[4];
         sq_v4f sc[4];
         operands(0);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            d[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[t >> 1], bf[t & 1], zero, 0, 0, 0);
+            d[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[t >> 1], bf[t & 1], ibase, 0, 0, 0);
             sc[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(sa[t >> 1], sw[t & 1], fzero, 0, 0, 0);
         }
 #pragma unroll
@@ -353,10 +375,10 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(MatView w, const int8_t*
                 for (int r = 0; r < 4; r++) {
                     // the combine of the reference's aarch64 kernels (dot_prod.rs:189-252):
                     // acc = fma(f32(isum), sa * sw, acc)
-                    acc[i][j][r] = fmaf((float)d[t][r], sc[t][r], acc[i][j][r]);
+                    acc[i][j][r] = fmaf(isum_f32(d[t][r]), sc[t][r], acc[i][j][r]);
                 }
                 if (b + 1 < MQ_KB) {
-                    d[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[i], bf[j], zero, 0, 0, 0);
+                    d[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[i], bf[j], ibase, 0, 0, 0);
                     sc[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(sa[i], sw[j], fzero, 0, 0, 0);
                 }
             }
@@ -394,9 +416,6 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(MatView w, const int8_t*
 constexpr int M8_KB = 2;           // blocks per chunk
 constexpr int M8_KC = M8_KB * 32;  // bytes per row per chunk
 constexpr int M8_LD = M8_KC + 16;  // LDS row stride: 16-byte reads of 8 consecutive rows cover all banks
-
-typedef int m8_v16i __attribute__((ext_vector_type(16)));
-typedef float m8_v16f __attribute__((ext_vector_type(16)));
 
 template <int BM, int BN>
 struct M8Loads {
@@ -516,6 +535,7 @@ __global__ __launch_bounds__(256, (m8_occupancy<BM, BN>())) void gemm_mfma32_ker
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
 
+    const m8_v16i ibase = isum_base<m8_v16i>();
     auto compute = [&](int buf) {
         const int8_t* A = sA[buf];
         const int8_t* W = sW[buf];
@@ -537,19 +557,18 @@ __global__ __launch_bounds__(256, (m8_occupancy<BM, BN>())) void gemm_mfma32_ker
         };
         // Products for (block, tile) pairs k = NT b + t, issued one pair ahead
         // of the pair being folded in.
-        const m8_v16i izero = {};
         const m8_v16f fzero = {};
         m8_v16i d[2];
         m8_v16f sc[2];
         operands(0);
-        d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[0], bf[0], izero, 0, 0, 0);
+        d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[0], bf[0], ibase, 0, 0, 0);
         sc[0] = __builtin_amdgcn_mfma_f32_32x32x8f16(sa[0], sw[0], fzero, 0, 0, 0);
 #pragma unroll
         for (int k = 0; k < NT * M8_KB; k++) {
             if (k + 1 < NT * M8_KB) {
                 const int t1 = (k + 1) % NT, i = t1 / SN, j = t1 % SN;
                 if (t1 == 0) operands((k + 1) / NT);
-                d[(k + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], izero, 0, 0, 0);
+                d[(k + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], ibase, 0, 0, 0);
                 sc[(k + 1) & 1] = __builtin_amdgcn_mfma_f32_32x32x8f16(sa[i], sw[j], fzero, 0, 0, 0);
             }
             // On 128 x 128 tiles the next pair's matrix instructions are kept
@@ -563,7 +582,7 @@ __global__ __launch_bounds__(256, (m8_occupancy<BM, BN>())) void gemm_mfma32_ker
             for (int r = 0; r < 16; r++) {
                 // the combine of the reference's aarch64 kernels (dot_prod.rs:189-252):
                 // acc = fma(f32(isum), sa * sw, acc)
-                acc[t][r] = fmaf((float)d[k & 1][r], sc[k & 1][r], acc[t][r]);
+                acc[t][r] = fmaf(isum_f32(d[k & 1][r]), sc[k & 1][r], acc[t][r]);
             }
             if constexpr (BN == 128) __builtin_amdgcn_sched_barrier(0);
         }
@@ -800,6 +819,7 @@ __global__ __launch_bounds__(256, (dma_occupancy<BM, BN>())) void gemm_dma_kerne
     for (int b = 0; b < SKB; b++) ua[b] = 16 * ((2 * b + fh) ^ dma_swz<SKB>(fr));
     const uint32_t lo_mask = fh ? 0u : 0xFFFFFFFFu;  // k-slots 4-7 (lanes 32-63) are zero
 
+    const m8_v16i ibase = isum_base<m8_v16i>();
     auto compute = [&](const Stage& S) {
         // scale operands: lanes 0-31 hold k-slots 0-3 of row (column) fr, the
         // others slots 4-7 (zero).  Block 2 d pairs (sa_{2d}, 0) with (sw_{2d},
@@ -824,7 +844,6 @@ __global__ __launch_bounds__(256, (dma_occupancy<BM, BN>())) void gemm_dma_kerne
             return __builtin_bit_cast(mq_v4h, make_uint2(v, 0u));
         };
         auto sw_op = [&](int b, int j) { return __builtin_bit_cast(mq_v4h, make_uint2(swr[b >> 1][j], 0u)); };
-        const m8_v16i izero = {};
         const m8_v16f fzero = {};
         if constexpr (BN == 128) {
             // (block, tile) pairs k = NT b + t in order, each pair's matrix
@@ -833,12 +852,12 @@ __global__ __launch_bounds__(256, (dma_occupancy<BM, BN>())) void gemm_dma_kerne
             for (int k = 0; k < NT * SKB; k++) {
                 const int t = k % NT, i = t / SN, j = t % SN, b = k / NT;
                 if (t == 0) operands(b);
-                const m8_v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], izero, 0, 0, 0);
+                const m8_v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], ibase, 0, 0, 0);
                 const m8_v16f sc = __builtin_amdgcn_mfma_f32_32x32x8f16(sa_op(b, i), sw_op(b, j), fzero, 0, 0, 0);
                 // the combine of the reference's aarch64 kernels (dot_prod.rs:189-252):
                 // acc = fma(f32(isum), sa * sw, acc)
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[t][r] = fmaf((float)d[r], sc[r], acc[t][r]);
+                for (int r = 0; r < 16; r++) acc[t][r] = fmaf(isum_f32(d[r]), sc[r], acc[t][r]);
             }
         } else {
             // the same pairs, each one's matrix instructions issued one pair
@@ -846,19 +865,19 @@ __global__ __launch_bounds__(256, (dma_occupancy<BM, BN>())) void gemm_dma_kerne
             m8_v16i d[2];
             m8_v16f sc[2];
             operands(0);
-            d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[0], bf[0], izero, 0, 0, 0);
+            d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[0], bf[0], ibase, 0, 0, 0);
             sc[0] = __builtin_amdgcn_mfma_f32_32x32x8f16(sa_op(0, 0), sw_op(0, 0), fzero, 0, 0, 0);
 #pragma unroll
             for (int k = 0; k < NT * SKB; k++) {
                 if (k + 1 < NT * SKB) {
                     const int t1 = (k + 1) % NT, i = t1 / SN, j = t1 % SN, b1 = (k + 1) / NT;
                     if (t1 == 0) operands(b1);
-                    d[(k + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], izero, 0, 0, 0);
+                    d[(k + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], ibase, 0, 0, 0);
                     sc[(k + 1) & 1] = __builtin_amdgcn_mfma_f32_32x32x8f16(sa_op(b1, i), sw_op(b1, j), fzero, 0, 0, 0);
                 }
                 const int t = k % NT;
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[t][r] = fmaf((float)d[k & 1][r], sc[k & 1][r], acc[t][r]);
+                for (int r = 0; r < 16; r++) acc[t][r] = fmaf(isum_f32(d[k & 1][r]), sc[k & 1][r], acc[t][r]);
             }
         }
     };
@@ -1190,7 +1209,7 @@ __global__ __launch_bounds__(RW_NW * 64) void gemm_rows_kernel(MatView w, const 
     for (int t = 0; t < NT; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
-    const m8_v16i izero = {};
+    const m8_v16i ibase = isum_base<m8_v16i>();
     const m8_v16f fzero = {};
     auto compute = [&](const Batch& B, int kb) {
 #pragma unroll
@@ -1220,10 +1239,10 @@ __global__ __launch_bounds__(RW_NW * 64) void gemm_rows_kernel(MatView w, const 
                 }
                 const uint16_t swv = inb && wvalid[t] ? (uint16_t)B.sw[t][j] : (uint16_t)0;
                 const mq_v4h sw = {__builtin_bit_cast(_Float16, swv), h0, h0, h0};
-                const m8_v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(B.a[j], wf, izero, 0, 0, 0);
+                const m8_v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(B.a[j], wf, ibase, 0, 0, 0);
                 const m8_v16f sc = __builtin_amdgcn_mfma_f32_32x32x8f16(sa, sw, fzero, 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[t][r] = fmaf((float)d[r], sc[r], acc[t][r]);
+                for (int r = 0; r < 16; r++) acc[t][r] = fmaf(isum_f32(d[r]), sc[r], acc[t][r]);
                 // one tile's products live at a time: left to itself the
                 // scheduler issues every block's matrix instructions first and
                 // spills their results
