@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "model.h"
+#include "scratch.h"
 
 namespace sq {
 
@@ -22,19 +23,6 @@ int synth_write(const std::string& path, const sq_synth_spec& s);
 using namespace sq;
 
 namespace {
-
-// Temporary device buffer for the operator-level entry points.
-struct Tmp {
-    void* p = nullptr;
-    ~Tmp() {
-        if (p) (void)hipFree(p);
-    }
-    int alloc(size_t n) {
-        hipError_t e = hipMalloc(&p, n ? n : 1);
-        if (e != hipSuccess) return set_error(SQ_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
-        return 0;
-    }
-};
 
 int finish(int st) {
     if (st) return st;
@@ -60,7 +48,12 @@ int sq_device_count(int* n) {
 }
 
 int sq_malloc(void** p, size_t bytes) {
-    SQ_HIP_CHECK(hipMalloc(p, bytes ? bytes : 1));
+    hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        scratch_trim();
+        SQ_HIP_CHECK(hipMalloc(p, bytes ? bytes : 1));
+    }
     return 0;
 }
 int sq_free(void* p) {
@@ -317,23 +310,11 @@ int sq_quantize_row_q8_0(const float* d_x, size_t n, void* d_blocks) {
 
 namespace {
 
-int linear_impl(const float* d_in, size_t m, size_t k, const sq_weight* w, float* d_out, uint32_t flags,
-                const int8_t* pre_q, const uint16_t* pre_d) {
-    if (!w || !d_in || !d_out) return set_error(SQ_ERR_ARG, "linear: null argument");
-    if (k != (size_t)w->m.k) return set_error(SQ_ERR_SHAPE, "linear: ShapeMismatch (in_dim != weight k)");
-    if (m == 0) return 0;
-    const bool a8 = w->m.wtype != WT_BF16 && !(flags & SQ_CTX_F32_ACTS);
-    if (!a8) return set_error(SQ_ERR_UNSUPPORTED, kA32Disabled);
-    Tmp tq, td;
-    int st;
-    const int8_t* aq = pre_q;
-    const uint16_t* ad = pre_d;
-    if (a8 && !aq) {
-        if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16))) return st;
-        if ((st = launch_quantize_rows(nullptr, d_in, m * k, (int8_t*)tq.p, (uint16_t*)td.p))) return st;
-        aq = (const int8_t*)tq.p;
-        ad = (const uint16_t*)td.p;
-    }
+// Launches the product of one weight with activations already quantized
+// (aq, ad); ws holds kGemmSplitFloats floats of partial tiles.
+int launch_linear(const float* d_in, size_t m, const sq_weight* w, float* d_out, const int8_t* aq, const uint16_t* ad,
+                  float* ws) {
+    const size_t k = w->m.k;
     if (m == 1 && (k / 32 <= 256)) {
         GemvArgs a{};
         a.w = view(w->m);
@@ -342,45 +323,50 @@ int linear_impl(const float* d_in, size_t m, size_t k, const sq_weight* w, float
         a.ad = ad;
         a.x = d_in;
         a.out = d_out;
-        st = launch_gemv(nullptr, a8 ? PRO_Q8 : PRO_F32, EPI_STORE, a8, a, nullptr);
-    } else {
-        Tmp ws;  // partial tiles of a K split
-        if ((st = ws.alloc(kGemmSplitFloats * sizeof(float)))) return st;
-        st = launch_gemm(nullptr, view(w->m), w->m.wtype, a8, aq, ad, d_in, (int)m, d_out, w->m.rows, false,
-                         (float*)ws.p, kGemmSplitFloats);
-        if (!st) st = finish(st);  // the workspace is freed on return
+        return launch_gemv(nullptr, PRO_Q8, EPI_STORE, true, a, nullptr);
     }
+    return launch_gemm(nullptr, view(w->m), w->m.wtype, true, aq, ad, d_in, (int)m, d_out, w->m.rows, false, ws,
+                       kGemmSplitFloats);
+}
+
+// Quantizes the m rows once (linear.rs:117-127), multiplies them with each
+// weight and waits once for all of it.
+int linear_all(const float* d_in, size_t m, size_t k, const sq_weight* const* ws, float* const* d_outs, size_t n) {
+    Tmp tq, td, split;
+    int st;
+    if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16))) return st;
+    if (!(m == 1 && (k / 32 <= 256)) && (st = split.alloc(kGemmSplitFloats * sizeof(float)))) return st;
+    st = launch_quantize_rows(nullptr, d_in, m * k, (int8_t*)tq.p, (uint16_t*)td.p);
+    for (size_t i = 0; i < n && !st; i++)
+        st = launch_linear(d_in, m, ws[i], d_outs[i], (const int8_t*)tq.p, (const uint16_t*)td.p, (float*)split.p);
     return finish(st);
 }
 
 }  // namespace
 
 int sq_linear(const float* d_in, size_t m, size_t k, const sq_weight* w, float* d_out, uint32_t flags) {
-    return linear_impl(d_in, m, k, w, d_out, flags, nullptr, nullptr);
+    if (!w || !d_in || !d_out) return set_error(SQ_ERR_ARG, "linear: null argument");
+    if (k != (size_t)w->m.k) return set_error(SQ_ERR_SHAPE, "linear: ShapeMismatch (in_dim != weight k)");
+    if (m == 0) return 0;
+    if (w->m.wtype == WT_BF16 || (flags & SQ_CTX_F32_ACTS)) return set_error(SQ_ERR_UNSUPPORTED, kA32Disabled);
+    return linear_all(d_in, m, k, &w, &d_out, 1);
 }
 
 int sq_linear_shared(const float* d_in, size_t m, size_t k, const sq_weight* const* ws, float* const* d_outs,
                      size_t n_weights, uint32_t flags) {
     if (n_weights == 0 || !ws || !d_outs) return set_error(SQ_ERR_SHAPE, "linear_shared: ShapeMismatch (no weights)");
+    if (!ws[0]) return set_error(SQ_ERR_ARG, "linear_shared: null weight");
     const int wt = ws[0]->m.wtype;
     for (size_t i = 0; i < n_weights; i++) {
         if (!ws[i]) return set_error(SQ_ERR_ARG, "linear_shared: null weight");
         if ((size_t)ws[i]->m.k != k) return set_error(SQ_ERR_SHAPE, "linear_shared: ShapeMismatch");
         if (ws[i]->m.wtype != wt) return set_error(SQ_ERR_INVALID_TYPE, "linear_shared: InvalidType (mixed types)");
     }
-    const bool a8 = wt != WT_BF16 && !(flags & SQ_CTX_F32_ACTS);
-    if (!a8) return set_error(SQ_ERR_UNSUPPORTED, kA32Disabled);
-    Tmp tq, td;
-    int st;
-    if (a8 && m) {
-        // One quantization shared by every projection (linear.rs:117-127).
-        if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16))) return st;
-        if ((st = launch_quantize_rows(nullptr, d_in, m * k, (int8_t*)tq.p, (uint16_t*)td.p))) return st;
-    }
+    if (wt == WT_BF16 || (flags & SQ_CTX_F32_ACTS)) return set_error(SQ_ERR_UNSUPPORTED, kA32Disabled);
     for (size_t i = 0; i < n_weights; i++)
-        if ((st = linear_impl(d_in, m, k, ws[i], d_outs[i], flags, (const int8_t*)tq.p, (const uint16_t*)td.p)))
-            return st;
-    return 0;
+        if (!d_in || !d_outs[i]) return set_error(SQ_ERR_ARG, "linear: null argument");
+    if (m == 0) return 0;
+    return linear_all(d_in, m, k, ws, d_outs, n_weights);
 }
 
 int sq_block_isums(const void* d_act_blocks, const sq_weight* w, size_t row, int32_t* d_isums) {

@@ -21,6 +21,7 @@
 // Prefill (n tokens): the same math over n rows with multi-row matmuls and a
 // tiled causal attention; only the last row feeds the LM head.
 #include "model.h"
+#include "scratch.h"
 
 #include <algorithm>
 #include <chrono>
@@ -90,6 +91,11 @@ template <typename T>
 int dmalloc(T** p, size_t count) {
     if (count == 0) count = 1;
     hipError_t e = hipMalloc((void**)p, count * sizeof(T));
+    if (e != hipSuccess) {  // the operators' idle scratch goes first
+        (void)hipGetLastError();
+        scratch_trim();
+        e = hipMalloc((void**)p, count * sizeof(T));
+    }
     if (e != hipSuccess)
         return set_error(SQ_ERR_HIP, "hipMalloc(" + std::to_string(count * sizeof(T)) + "): " + hipGetErrorString(e));
     return 0;

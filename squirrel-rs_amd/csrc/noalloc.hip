@@ -1,7 +1,7 @@
 // sq_linear_noalloc: the linear operator with no device allocation.
 //
-// sq_linear allocates its scratch (the Q8_0 activation payload and block
-// scales, and the partial tiles of a K split) with hipMalloc on every call.
+// sq_linear takes its scratch (the Q8_0 activation payload and block scales,
+// and the partial tiles of a K split) from a pool that grows with hipMalloc.
 // Callers that cannot allocate -- tight serving loops, harnesses that forbid
 // it -- use this variant: its scratch is one
 // file-scope device array, `scratch`, held by each GPU the library runs on

@@ -551,6 +551,38 @@ def test_log_softmax_at_closed_forms():
         ls(x, 128256)
 
 
+def test_linear_from_several_threads():
+    """Calls share a pool of scratch blocks: threads that multiply inputs of
+    different sizes at once, over and over, each get the results of a call
+    made alone, bit for bit."""
+    import threading
+    cases = []
+    for i, (m, k, n) in enumerate([(1, 2048, 512), (9, 512, 300), (40, 1024, 256), (130, 256, 2048)]):
+        w, _ = quant_weights(O.Q8_0, n, k, seed=40 + i)
+        W = ops.Weight(O.Q8_0, w, n, k)
+        x = DeviceArray.from_numpy((rng(i).standard_normal((m, k))).astype(np.float32))
+        alone = DeviceArray((m, n))
+        ops.linear(x, W, alone)
+        cases.append((W, x, alone.numpy(), [DeviceArray((m, n)) for _ in range(12)]))
+    errors = []
+
+    def work(W, x, want, outs):
+        try:
+            for o in outs:
+                ops.linear(x, W, o)
+            for o in outs:
+                assert np.array_equal(o.numpy(), want)
+        except BaseException as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=c) for c in cases]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+
+
 @pytest.mark.parametrize("n", [1, 255, 2047, 2048, 2049, 4097, 512 * 2048 + 5])
 def test_log_softmax_at_chunk_edges(n):
     """Rows of one partial chunk, whole chunks and chunks longer than the
