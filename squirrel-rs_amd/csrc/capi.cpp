@@ -434,17 +434,11 @@ int sq_sdpa(const float* d_q, const float* d_k, const float* d_v, float* d_out, 
     int st;
     if (model_kernels && seq_q == 1) {
         // The decode kernel: the query sits at position seq_k - 1.
-        const int tiles = (int)((seq_k + 63) / 64);
-        Tmp pos, pm, pl, po, cnt, aq, ad;
-        const int p = (int)seq_k - 1;
-        if ((st = pos.alloc(4)) || (st = pm.alloc(n_heads * tiles * 4)) || (st = pl.alloc(n_heads * tiles * 4)) ||
-            (st = po.alloc(n_heads * tiles * 64 * 4)) || (st = cnt.alloc(n_kv_heads * 4)))
-            return st;
-        SQ_HIP_CHECK(hipMemcpy(pos.p, &p, 4, hipMemcpyHostToDevice));
-        SQ_HIP_CHECK(hipMemset(cnt.p, 0, n_kv_heads * 4));
-        return finish(launch_attn_decode(nullptr, d_q, d_k, d_v, (const int*)pos.p, (int)n_heads, (int)n_kv_heads, 64,
-                                         tiles, (float*)pm.p, (float*)pl.p, (float*)po.p, (unsigned*)cnt.p, d_out,
-                                         nullptr, nullptr));
+        Tmp ws;
+        const size_t floats = attn_decode_floats((int)seq_k, (int)n_heads);
+        if (floats && (st = ws.alloc(floats * sizeof(float)))) return st;
+        return finish(launch_attn_decode_at(nullptr, d_q, d_k, d_v, (int)seq_k, (int)n_heads, (int)n_kv_heads, 64,
+                                            (float*)ws.p, d_out));
     }
     if (model_kernels) {
         Tmp kvs;

@@ -24,69 +24,148 @@ inline int check_launch(const char* what) {
     return 0;
 }
 
-// Decode attention.  One workgroup per (kv head, tile of 64 positions): the
-// tile's K and V rows are staged in LDS with one coalesced load round, the G
-// query heads sharing the kv head (GQA) score all 64 positions in parallel,
-// and each head's tile partial (running max m, sum l, unnormalized P*V) goes
-// to global memory.  The workgroup that finishes last for a kv head (device
-// fence + atomic counter) merges the tiles with the log-sum-exp rule, writes
-// the attention output and, for the integer path, its Q8_0 blocks (the
-// reference quantizes this row inside the o-projection's `linear`,
-// src/kernels/matmul.rs:91-98).  Tiles beyond the current length exit at
-// once, so one launch shape serves every position of a captured graph.
+// Decode attention.  One workgroup per (kv head, tile of 64 positions).  All
+// of a thread's K and V loads are issued first: for the scores it holds a
+// quarter of one position's K row (the lane quad of a position adds its four
+// partial dots through DPP), for the output four dimensions of four positions'
+// V rows, so neither tile passes through LDS (staged there, the scores alone
+// read 128 words of it per thread: 37 us for 32 heads over 4096 keys, with the
+// merge below, against 4.6 + 3.4 now).  Each head's tile partial (running max m, sum
+// l, unnormalized P*V) goes to global memory and the tiles are merged with the
+// log-sum-exp rule, by attn_merge_kernel or, with LAST, by the workgroup that
+// finishes last for a kv head (device fence + atomic counter: one launch shape
+// then serves every position of a captured graph; tiles beyond the current
+// length exit at once).  A single tile writes the output itself.  For the
+// integer path the row's Q8_0 blocks are written too (the reference quantizes
+// this row inside the o-projection's `linear`, src/kernels/matmul.rs:91-98).
 constexpr int TP = 64;  // positions per tile
 
-template <int G>
+// The output of head h at dimension `lane` (every lane of the wavefront active).
+__device__ __forceinline__ void attn_decode_store(float out, int h, int lane, float* attn, int8_t* act_q,
+                                                  uint16_t* act_d) {
+    attn[h * HD + lane] = out;
+    if (act_q) {
+        const float amax = fmaxf(sq_half_max(fabsf(out)), 0.0f);
+        const float sc = sq_q8_scale(amax);
+        const float inv = sq_q8_inv(sc);
+        act_q[h * HD + lane] = sq_q8_quant(out, inv);
+        if ((lane & 31) == 0) act_d[(h * HD + lane) >> 5] = sq_f32_to_f16(sc);
+    }
+}
+
+// One wavefront's part of the merge of a head's ntiles partials (pm, pl, po):
+// dimension `lane` of the sum over the tiles w, w + NW, ..., rescaled to the
+// maximum over all tiles, and the whole sum L (the same on every wavefront).
+// Sixteen tiles' outputs are in flight at a time (64 with NW = 4).
+template <int NW>
+__device__ __forceinline__ float attn_merge_part(const float* pm, const float* pl, const float* po, int ntiles, int w,
+                                                 int lane, float& L) {
+    float M = -INFINITY;
+    for (int t = lane; t < ntiles; t += 64) M = fmaxf(M, pm[t]);
+    M = sq_wave_max(M);
+    float l = 0.0f, O = 0.0f;
+    for (int c = 0; c < ntiles; c += 64) {
+        const int t = c + lane;
+        const float mt = t < ntiles ? pm[t] : -INFINITY;
+        // a tile whose every score is -inf is left out (-1)
+        const float e = mt == -INFINITY ? -1.0f : expf(mt - M);
+        if (mt != -INFINITY) l += pl[t] * e;
+        const int n = min(64, ntiles - c);
+        for (int k0 = w; k0 < n; k0 += 16 * NW) {
+            float v[16];
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int tt = min(k0 + k * NW, n - 1);
+                v[k] = po[(size_t)(c + tt) * HD + lane];
+            }
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int tt = k0 + k * NW;
+                const float et = __shfl(e, min(tt, 63), 64);
+                if (tt < n && et != -1.0f) O += v[k] * et;
+            }
+        }
+    }
+    L = sq_wave_sum(l);
+    return O;
+}
+
+__global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict__ part_m,
+                                                         const float* __restrict__ part_l,
+                                                         const float* __restrict__ part_o, int ntiles, int max_tiles,
+                                                         float* attn, int8_t* act_q, uint16_t* act_d) {
+    __shared__ float s_o[4][HD];
+    const int h = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const size_t p = (size_t)h * max_tiles;
+    float L;
+    s_o[wave][lane] = attn_merge_part<4>(part_m + p, part_l + p, part_o + p * HD, ntiles, wave, lane, L);
+    __syncthreads();
+    if (wave == 0)
+        attn_decode_store(((s_o[0][lane] + s_o[1][lane]) + (s_o[2][lane] + s_o[3][lane])) / L, h, lane, attn, act_q,
+                          act_d);
+}
+
+template <int G, bool LAST>
 __global__ __launch_bounds__(256) void attn_decode_kernel(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-    const int* __restrict__ pos_ptr, int n_kv_heads, int max_tiles, float* part_m, float* part_l,
+    const int* __restrict__ pos_ptr, int pos_value, int n_kv_heads, int max_tiles, float* part_m, float* part_l,
     float* part_o, unsigned* counters, float* attn, int8_t* act_q, uint16_t* act_d) {
-    __shared__ float s_k[TP][HD + 1];
-    __shared__ __attribute__((aligned(16))) float s_v[TP][HD];
-    __shared__ float s_q[G][HD];
+    __shared__ __attribute__((aligned(16))) float s_q[G][HD];
     __shared__ float s_p[G][TP];
     __shared__ float s_m[G], s_l[G];
+    __shared__ __attribute__((aligned(16))) float s_o[16][G][HD];  // per group of four positions
     __shared__ int s_last;
     const int g = blockIdx.x;
     const int tile = blockIdx.y;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int P = *pos_ptr + 1;
+    const int P = (pos_ptr ? *pos_ptr : pos_value) + 1;
     const int ntiles = (P + TP - 1) / TP;
     if (tile >= ntiles) return;
     const int kv_dim = n_kv_heads * HD;
     const int s0 = tile * TP;
     const float scale = 1.0f / sqrtf((float)HD);
 
-    for (int e = tid; e < TP * HD / 4; e += 256) {
-        const int r = e / (HD / 4), c4 = e % (HD / 4);
-        float4 k4 = make_float4(0.f, 0.f, 0.f, 0.f), v4 = k4;
-        if (s0 + r < P) {
-            const size_t off = (size_t)(s0 + r) * kv_dim + g * HD + 4 * c4;
-            k4 = *(const float4*)(kc + off);
-            v4 = *(const float4*)(vc + off);
-        }
-        s_k[r][4 * c4 + 0] = k4.x;
-        s_k[r][4 * c4 + 1] = k4.y;
-        s_k[r][4 * c4 + 2] = k4.z;
-        s_k[r][4 * c4 + 3] = k4.w;
-        *(float4*)&s_v[r][4 * c4] = v4;
+    // Positions past the last read the last one; their scores are masked and
+    // their V is set to zero (0 times an infinite value would be NaN).
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    const int sp = tid >> 2, qd = tid & 3;   // scores: position s0 + sp, dims 16 c + 4 qd ..
+    const int pg = tid >> 4, d4 = tid & 15;  // output: positions s0 + pg + 16 j, dims 4 d4 ..
+    v4f k[4], v[4];
+    const float* kr = kc + (size_t)min(s0 + sp, P - 1) * kv_dim + g * HD + 4 * qd;
+#pragma unroll
+    for (int c = 0; c < 4; c++) k[c] = *(const v4f*)(kr + 16 * c);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        v[j] = *(const v4f*)(vc + (size_t)min(s0 + pg + 16 * j, P - 1) * kv_dim + g * HD + 4 * d4);
+    if (s0 + TP > P) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (s0 + pg + 16 * j >= P) v[j] = v4f{0.f, 0.f, 0.f, 0.f};
     }
     for (int e = tid; e < G * HD; e += 256) s_q[e / HD][e % HD] = q[(size_t)g * G * HD + e];
     __syncthreads();
 
     // scores = dot(q, k) * (1/sqrt(head_dim)) (attention.rs:52-55)
-    for (int idx = tid; idx < G * TP; idx += 256) {
-        const int i = idx / TP, sp = idx % TP;
+#pragma unroll
+    for (int i = 0; i < G; i++) {
         float dot = 0.0f;
-#pragma unroll 16
-        for (int d = 0; d < HD; d++) dot += s_q[i][d] * s_k[sp][d];
-        s_p[i][sp] = (s0 + sp < P) ? dot * scale : -INFINITY;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const v4f qv = *(const v4f*)&s_q[i][16 * c + 4 * qd];
+            dot += qv.x * k[c].x;
+            dot += qv.y * k[c].y;
+            dot += qv.z * k[c].z;
+            dot += qv.w * k[c].w;
+        }
+        dot += sq_dpp<0xB1, 0xF>(dot);  // the lane quad's four quarters
+        dot += sq_dpp<0x4E, 0xF>(dot);
+        if (qd == (i & 3)) s_p[i][sp] = (s0 + sp < P) ? dot * scale : -INFINITY;
     }
     __syncthreads();
     for (int i = wave; i < G; i += 4) {
-        const float v = s_p[i][lane];
-        const float m = sq_wave_max(v);
-        const float p = (v == -INFINITY) ? 0.0f : expf(v - m);
+        const float x = s_p[i][lane];
+        const float m = sq_wave_max(x);
+        const float p = (x == -INFINITY) ? 0.0f : expf(x - m);
         const float l = sq_wave_sum(p);
         s_p[i][lane] = p;
         if (lane == 0) {
@@ -95,52 +174,50 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
         }
     }
     __syncthreads();
-    for (int idx = tid; idx < G * HD; idx += 256) {
-        const int i = idx / HD, d = idx % HD;
-        float o = 0.0f;
-#pragma unroll 16
-        for (int sp = 0; sp < TP; sp++) o += s_p[i][sp] * s_v[sp][d];
-        const int pidx = (g * G + i) * max_tiles + tile;
-        part_o[(size_t)pidx * HD + d] = o;
-        if (d == 0) {
-            part_m[pidx] = s_m[i];
-            part_l[pidx] = s_l[i];
-        }
-    }
-
-    __syncthreads();
-    if (tid == 0) {
-        __threadfence();
-        const unsigned prev = atomicAdd(&counters[g], 1u);
-        s_last = prev == (unsigned)(ntiles - 1);
+#pragma unroll
+    for (int i = 0; i < G; i++) {
+        v4f o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; j++) o += s_p[i][pg + 16 * j] * v[j];
+        *(v4f*)&s_o[pg][i][4 * d4] = o;
     }
     __syncthreads();
-    if (!s_last) return;
-    __threadfence();
-    for (int idx = tid; idx < G * HD; idx += 256) {
+    for (int idx = tid; idx < G * HD; idx += 256) {  // whole wavefronts: one head each
         const int i = idx / HD, d = idx % HD, h = g * G + i;
-        float M = -INFINITY;
-        for (int t = 0; t < ntiles; t++) M = fmaxf(M, part_m[h * max_tiles + t]);
-        float L = 0.0f, O = 0.0f;
-        for (int t = 0; t < ntiles; t++) {
-            const int pidx = h * max_tiles + t;
-            const float mt = part_m[pidx];
-            if (mt == -INFINITY) continue;
-            const float e = expf(mt - M);
-            L += part_l[pidx] * e;
-            O += part_o[(size_t)pidx * HD + d] * e;
-        }
-        const float out = O / L;
-        attn[h * HD + d] = out;
-        if (act_q) {
-            const float amax = fmaxf(sq_half_max(fabsf(out)), 0.0f);
-            const float sc = sq_q8_scale(amax);
-            const float inv = sq_q8_inv(sc);
-            act_q[h * HD + d] = sq_q8_quant(out, inv);
-            if ((d & 31) == 0) act_d[(h * HD + d) >> 5] = sq_f32_to_f16(sc);
+        float o = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) o += s_o[r][i][d];
+        if (ntiles == 1) {
+            attn_decode_store(o / s_l[i], h, d, attn, act_q, act_d);
+        } else {
+            const size_t pidx = (size_t)h * max_tiles + tile;
+            part_o[pidx * HD + d] = o;
+            if (d == 0) {
+                part_m[pidx] = s_m[i];
+                part_l[pidx] = s_l[i];
+            }
         }
     }
-    if (tid == 0) atomicExch(&counters[g], 0u);
+    if constexpr (LAST) {
+        if (ntiles == 1) return;
+        __syncthreads();
+        if (tid == 0) {
+            __threadfence();
+            const unsigned prev = atomicAdd(&counters[g], 1u);
+            s_last = prev == (unsigned)(ntiles - 1);
+        }
+        __syncthreads();
+        if (!s_last) return;
+        __threadfence();
+        for (int i = wave; i < G; i += 4) {
+            const int h = g * G + i;
+            const size_t p = (size_t)h * max_tiles;
+            float L;
+            const float O = attn_merge_part<1>(part_m + p, part_l + p, part_o + p * HD, ntiles, 0, lane, L);
+            attn_decode_store(O / L, h, lane, attn, act_q, act_d);
+        }
+        if (tid == 0) atomicExch(&counters[g], 0u);
+    }
 }
 
 // Prefill attention on the matrix cores, f32 in and out
@@ -826,16 +903,19 @@ bool attn_use_f32(int n_keys) {
 
 }  // namespace
 
-int launch_attn_decode(hipStream_t s, const float* q, const float* kcache, const float* vcache, const int* pos,
-                       int n_heads, int n_kv_heads, int head_dim, int max_tiles, float* part_m, float* part_l,
-                       float* part_o, unsigned* counters, float* attn, int8_t* act_q, uint16_t* act_d) {
-    if (head_dim != HD) return set_error(SQ_ERR_UNSUPPORTED, "attention kernels are built for head_dim 64");
-    const int G = n_heads / n_kv_heads;
-    dim3 grid(n_kv_heads, max_tiles);
-#define SQ_ATTN_LAUNCH(GG)                                                                                      \
-    hipLaunchKernelGGL(attn_decode_kernel<GG>, grid, dim3(256), 0, s, q, kcache, vcache, pos, n_kv_heads,      \
-                       max_tiles, part_m, part_l, part_o, counters, attn, act_q, act_d)
-    switch (G) {
+// The decode attention of one position over `tiles` tiles (at most max_tiles
+// partials per head): pos is null where the host knows the position
+// (pos_value), and the merge is then a launch of its own.
+template <bool LAST>
+static int run_attn_decode(hipStream_t s, const float* q, const float* kcache, const float* vcache, const int* pos,
+                           int pos_value, int n_heads, int n_kv_heads, int tiles, int max_tiles, float* part_m,
+                           float* part_l, float* part_o, unsigned* counters, float* attn, int8_t* act_q,
+                           uint16_t* act_d) {
+    const dim3 grid(n_kv_heads, tiles);
+#define SQ_ATTN_LAUNCH(GG)                                                                                          \
+    hipLaunchKernelGGL((attn_decode_kernel<GG, LAST>), grid, dim3(256), 0, s, q, kcache, vcache, pos, pos_value,    \
+                       n_kv_heads, max_tiles, part_m, part_l, part_o, counters, attn, act_q, act_d)
+    switch (n_heads / n_kv_heads) {
         case 1: SQ_ATTN_LAUNCH(1); break;
         case 2: SQ_ATTN_LAUNCH(2); break;
         case 4: SQ_ATTN_LAUNCH(4); break;
@@ -844,6 +924,35 @@ int launch_attn_decode(hipStream_t s, const float* q, const float* kcache, const
     }
 #undef SQ_ATTN_LAUNCH
     return check_launch("attn_decode");
+}
+
+int launch_attn_decode(hipStream_t s, const float* q, const float* kcache, const float* vcache, const int* pos,
+                       int n_heads, int n_kv_heads, int head_dim, int max_tiles, float* part_m, float* part_l,
+                       float* part_o, unsigned* counters, float* attn, int8_t* act_q, uint16_t* act_d) {
+    if (head_dim != HD) return set_error(SQ_ERR_UNSUPPORTED, "attention kernels are built for head_dim 64");
+    return run_attn_decode<true>(s, q, kcache, vcache, pos, 0, n_heads, n_kv_heads, max_tiles, max_tiles, part_m,
+                                 part_l, part_o, counters, attn, act_q, act_d);
+}
+
+size_t attn_decode_floats(int n_keys, int n_heads) {
+    const size_t tiles = ((size_t)n_keys + TP - 1) / TP;
+    return tiles > 1 ? (size_t)n_heads * tiles * (HD + 2) : 0;
+}
+
+int launch_attn_decode_at(hipStream_t s, const float* q, const float* k, const float* v, int n_keys, int n_heads,
+                          int n_kv_heads, int head_dim, float* ws, float* out) {
+    if (head_dim != HD) return set_error(SQ_ERR_UNSUPPORTED, "attention kernels are built for head_dim 64");
+    const int tiles = (n_keys + TP - 1) / TP;
+    const size_t n = (size_t)n_heads * tiles;
+    float* const pm = ws ? ws + n * HD : nullptr;
+    float* const pl = ws ? pm + n : nullptr;
+    if (const int st = run_attn_decode<false>(s, q, k, v, nullptr, n_keys - 1, n_heads, n_kv_heads, tiles, tiles, pm, pl,
+                                              ws, nullptr, out, nullptr, nullptr))
+        return st;
+    if (tiles == 1) return 0;
+    hipLaunchKernelGGL(attn_merge_kernel, dim3(n_heads), dim3(256), 0, s, pm, pl, ws, tiles, tiles, out,
+                       (int8_t*)nullptr, (uint16_t*)nullptr);
+    return check_launch("attn_merge");
 }
 
 size_t attn_split_words(int max_keys, int n_kv_heads) {

@@ -73,6 +73,11 @@ int launch_attn_decode(hipStream_t s, const float* q, const float* kcache, const
                        const int* pos, int n_heads, int n_kv_heads, int head_dim, int max_tiles,
                        float* part_m, float* part_l, float* part_o, unsigned* counters, float* attn,
                        int8_t* act_q, uint16_t* act_d);
+// The same over k and v rows 0 .. n_keys - 1, the length known to the host.
+// ws: attn_decode_floats(n_keys, n_heads) floats (null where that is 0).
+size_t attn_decode_floats(int n_keys, int n_heads);
+int launch_attn_decode_at(hipStream_t s, const float* q, const float* k, const float* v, int n_keys, int n_heads,
+                          int n_kv_heads, int head_dim, float* ws, float* out);
 // Prefill: m query rows at positions pos0 .. pos0+m-1 against keys 0..pos0+m-1.
 // Writes the rows to out and/or, when act_q is non-null, their Q8_0 blocks
 // ([m][n_heads*64] and [m][n_heads*2]: what launch_quantize_rows makes of

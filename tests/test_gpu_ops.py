@@ -449,6 +449,29 @@ def test_sdpa_model_kernels_match_oracle(seq_q, seq_k, nh, nkv, attn, monkeypatc
     assert np.allclose(got, want, rtol=1e-5, atol=2e-6), float(np.abs(got - want).max())
 
 
+@pytest.mark.parametrize("seq_k", [2, 63, 64, 65, 128, 129, 1000, 4095, 4097, 8200])
+@pytest.mark.parametrize("nh,nkv", [(32, 8), (4, 2), (8, 1), (3, 3)])
+def test_sdpa_decode_tile_edges(seq_k, nh, nkv):
+    """One query over key counts around the 64-position tiles, the merge's 64
+    tiles per round and its 16 loads in flight, for every GQA group size;
+    an infinite V row past the keys (the same buffer's next row) is not read
+    into the result.  The bound of the test above: outputs are convex
+    combinations of v rows."""
+    hd = 64
+    r = rng(seq_k + nh)
+    q = r.standard_normal(nh * hd).astype(np.float32) * 2
+    k = r.standard_normal(seq_k * nkv * hd).astype(np.float32)
+    v = r.standard_normal(seq_k * nkv * hd).astype(np.float32)
+    st, want = O.sdpa(q, k, v, 1, seq_k, nh, nkv, hd)
+    assert st == 0
+    got = sdpa_dev(q, k, v, 1, seq_k, nh, nkv, hd)
+    assert np.allclose(got, want, rtol=1e-5, atol=2e-6), float(np.abs(got - want).max())
+    # an infinite last row reaches the output as infinities, not NaN
+    v[-nkv * hd:] = np.inf
+    got = sdpa_dev(q, k, v, 1, seq_k, nh, nkv, hd)
+    assert np.all(np.isposinf(got))
+
+
 @pytest.mark.parametrize("scale", [1e-3, 1.0, 6.0])
 def test_prefill_attention_split_f16_within_f32_noise(scale, monkeypatch):
     """The prefill attention's split-f16 products (hi + 2^-11 lo halves of
