@@ -281,7 +281,7 @@ int sq_weight_upload(int wtype, const void* blocks, size_t rows, size_t k, sq_we
         return set_error(SQ_ERR_INVALID_TYPE, "weight_upload: InvalidType");
     if (k == 0 || k % 32) return set_error(SQ_ERR_SHAPE, "weight_upload: k must be a multiple of 32");
     sq_weight* w = new sq_weight();
-    int st = upload_matrix(wtype, (const uint8_t*)blocks, rows, k, &w->m);
+    int st = upload_matrix(wtype, (const uint8_t*)blocks, rows, k, &w->m, true);
     if (st) {
         free_matrix(&w->m);
         delete w;
@@ -303,7 +303,7 @@ int sq_quantize_row_q8_0(const float* d_x, size_t n, void* d_blocks) {
     Tmp qs, d;
     int st;
     if ((st = qs.alloc(n)) || (st = d.alloc(n / 16))) return st;
-    if ((st = launch_quantize_rows(nullptr, d_x, n, (int8_t*)qs.p, (uint16_t*)d.p))) return st;
+    if ((st = launch_quantize_rows(nullptr, d_x, 1, n, (int8_t*)qs.p, (uint16_t*)d.p))) return st;
     st = launch_pack_q8_blocks(nullptr, (int8_t*)qs.p, (uint16_t*)d.p, n / 32, d_blocks);
     return finish(st);
 }
@@ -325,7 +325,7 @@ int launch_linear(const float* d_in, size_t m, const sq_weight* w, float* d_out,
         a.out = d_out;
         return launch_gemv(nullptr, PRO_Q8, EPI_STORE, true, a, nullptr);
     }
-    return launch_gemm(nullptr, view(w->m), w->m.wtype, true, aq, ad, d_in, (int)m, d_out, w->m.rows, false, ws,
+    return launch_gemm(nullptr, w->m, true, aq, ad, d_in, (int)m, d_out, w->m.rows, false, ws,
                        kGemmSplitFloats);
 }
 
@@ -336,7 +336,7 @@ int linear_all(const float* d_in, size_t m, size_t k, const sq_weight* const* ws
     int st;
     if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16))) return st;
     if (!(m == 1 && (k / 32 <= 256)) && (st = split.alloc(kGemmSplitFloats * sizeof(float)))) return st;
-    st = launch_quantize_rows(nullptr, d_in, m * k, (int8_t*)tq.p, (uint16_t*)td.p);
+    st = launch_quantize_rows(nullptr, d_in, m, k, (int8_t*)tq.p, (uint16_t*)td.p);
     for (size_t i = 0; i < n && !st; i++)
         st = launch_linear(d_in, m, ws[i], d_outs[i], (const int8_t*)tq.p, (const uint16_t*)td.p, (float*)split.p);
     return finish(st);

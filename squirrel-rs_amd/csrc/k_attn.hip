@@ -81,7 +81,8 @@ __device__ __forceinline__ float attn_merge_part(const float* pm, const float* p
 #pragma unroll
             for (int k = 0; k < 16; k++) {
                 const int tt = k0 + k * NW;
-                const float et = __shfl(e, min(tt, 63), 64);
+                const float et = __builtin_bit_cast(
+                    float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), __builtin_amdgcn_readfirstlane(min(tt, 63))));
                 if (tt < n && et != -1.0f) O += v[k] * et;
             }
         }
@@ -462,9 +463,10 @@ __global__ __launch_bounds__(256, 3) void attn_prefill_kernel(const float* __res
                     unsigned wq = 0;
 #pragma unroll
                     for (int c = 0; c < 4; c++) wq |= (unsigned)(uint8_t)sq_q8_quant(y[dt][c], qinv) << (8 * c);
-                    *(unsigned*)(act_q + (size_t)tq * q_dim + h * HD + 16 * dt + 4 * lk) = wq;
+                    *(unsigned*)(act_q + frag_q8(m_rows, q_dim, tq, h * (HD / 32) + b) +
+                                 (size_t)(dt & 1) * 16 * frag_tile_rows(m_rows, tq) + 4 * lk) = wq;
                 }
-                if (lk == 0) act_d[(size_t)tq * (q_dim / 32) + h * (HD / 32) + b] = sq_f32_to_f16(scale);
+                if (lk == 0) act_d[frag_scale(m_rows, q_dim / 32, tq, h * (HD / 32) + b)] = sq_f32_to_f16(scale);
             }
         }
     }
@@ -837,9 +839,10 @@ __global__ __launch_bounds__(256, 4) void attn_prefill_split_kernel(const float*
                     unsigned wq = 0;
 #pragma unroll
                     for (int c = 0; c < 4; c++) wq |= (unsigned)(uint8_t)sq_q8_quant(y[dt][c], qinv) << (8 * c);
-                    *(unsigned*)(act_q + (size_t)tq * q_dim + h * HD + 16 * dt + 4 * lk) = wq;
+                    *(unsigned*)(act_q + frag_q8(m_rows, q_dim, tq, h * (HD / 32) + b) +
+                                 (size_t)(dt & 1) * 16 * frag_tile_rows(m_rows, tq) + 4 * lk) = wq;
                 }
-                if (lk == 0) act_d[(size_t)tq * (q_dim / 32) + h * (HD / 32) + b] = sq_f32_to_f16(scale);
+                if (lk == 0) act_d[frag_scale(m_rows, q_dim / 32, tq, h * (HD / 32) + b)] = sq_f32_to_f16(scale);
             }
         }
     }

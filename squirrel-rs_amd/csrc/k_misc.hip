@@ -53,37 +53,45 @@ __global__ __launch_bounds__(kBlock) void embed_kernel(MatView table, const uint
     }
 }
 
-// rms_norm over rows (src/ops/rms_norm.rs:13-43); when act_q is non-null the
-// normed row is also quantized to Q8_0 (quantize_row_q8_0, dot_prod.rs:21-31).
-// Defined below the Q8_0 emitter it uses.
-__global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(const float* x, const float* w, int dim,
-                                                               float eps, float* out, int8_t* act_q,
-                                                               uint16_t* act_d);
+// Row and column of element (or group) g of rows of k: 32-bit division where
+// the count n fits.
+__device__ __forceinline__ void row_col(size_t g, size_t n, size_t k, int& row, size_t& col) {
+    const size_t r = n >> 32 ? g / k : (size_t)((uint32_t)g / (uint32_t)k);
+    row = (int)r;
+    col = g - r * k;
+}
 
-// quantize_row_q8_0 over n values (n a multiple of 32): one block per 32 lanes.
-__global__ __launch_bounds__(kBlock) void quantize_kernel(const float* x, size_t n, int8_t* qs,
+// quantize_row_q8_0 over m rows of k values (k a multiple of 32) into
+// fragment order: one block per 32 lanes.
+__global__ __launch_bounds__(kBlock) void quantize_kernel(const float* x, int m, size_t k, int8_t* qs,
                                                            uint16_t* d) {
-    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x, n = (size_t)m * k;
     const bool vi = i < n;
     const float v = vi ? x[i] : 0.0f;
     float amax = fmaxf(sq_half_max(fabsf(v)), 0.0f);
     float scale = sq_q8_scale(amax);
     float inv = sq_q8_inv(scale);
     if (vi) {
-        qs[i] = sq_q8_quant(v, inv);
-        if ((i & 31) == 0) d[i >> 5] = sq_f32_to_f16(scale);
+        int row;
+        size_t c;
+        row_col(i, n, k, row, c);
+        const int kb = (int)(c >> 5), e = (int)(c & 31);
+        qs[frag_q8(m, (int)k, row, kb) + (size_t)(e >> 4) * 16 * frag_tile_rows(m, row) + (e & 15)] = sq_q8_quant(v, inv);
+        if (e == 0) d[frag_scale(m, (int)(k >> 5), row, kb)] = sq_f32_to_f16(scale);
     }
 }
 
 // Q8_0 blocks of 8 consecutive values per thread (a lane quad holds a
-// block): the quantizer above with 16-byte loads and 8-byte stores.  All
+// block), into fragment order: the quantizer above with 16-byte loads and
+// 8-byte stores.  t8: the group's index in row `row` of m rows of k.  All
 // values of one 32-element block are quantized with the same scale, so the
 // result is that of quantize_kernel.
-__device__ __forceinline__ void q8_emit8(const float* v, size_t g, bool valid, int8_t* qs, uint16_t* d) {
-    float m = 0.0f;
+__device__ __forceinline__ void q8_emit8(const float* v, int m, int k, int row, int t8, bool valid, int8_t* qs,
+                                         uint16_t* d) {
+    float mx = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 8; e++) m = fmaxf(m, fabsf(v[e]));
-    const float amax = fmaxf(sq_quad_max(m), 0.0f);
+    for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf(v[e]));
+    const float amax = fmaxf(sq_quad_max(mx), 0.0f);
     const float scale = sq_q8_scale(amax), inv = sq_q8_inv(scale);
     if (valid) {
         unsigned lo = 0, hi = 0;
@@ -92,24 +100,132 @@ __device__ __forceinline__ void q8_emit8(const float* v, size_t g, bool valid, i
             lo |= (unsigned)(uint8_t)sq_q8_quant(v[e], inv) << (8 * e);
             hi |= (unsigned)(uint8_t)sq_q8_quant(v[e + 4], inv) << (8 * e);
         }
-        *(uint2*)(qs + 8 * g) = make_uint2(lo, hi);
-        if ((g & 3) == 0) d[g >> 2] = sq_f32_to_f16(scale);
+        const int kb = t8 >> 2, part = t8 & 3;  // eight bytes `part` of block kb
+        const size_t o = frag_q8(m, k, row, kb) + (size_t)(part >> 1) * 16 * frag_tile_rows(m, row) + 8 * (part & 1);
+        *(uint2*)(qs + o) = make_uint2(lo, hi);
+        if (part == 0) d[frag_scale(m, k >> 5, row, kb)] = sq_f32_to_f16(scale);
     }
 }
 
-__global__ __launch_bounds__(kBlock) void quantize8_kernel(const float* __restrict__ x, size_t n8,
+__global__ __launch_bounds__(kBlock) void quantize8_kernel(const float* __restrict__ x, int m, size_t k,
                                                             int8_t* __restrict__ qs, uint16_t* __restrict__ d) {
-    const size_t g = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    const size_t g = (size_t)blockIdx.x * kBlock + threadIdx.x, n8 = (size_t)m * k / 8;
     const bool vg = g < n8;
     float v[8] = {};
+    int row = 0;
+    size_t t8 = 0;
     if (vg) {
         const float4 a = ((const float4*)x)[2 * g], b = ((const float4*)x)[2 * g + 1];
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
         v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        row_col(g, n8, k / 8, row, t8);
     }
-    q8_emit8(v, g, vg, qs, d);
+    q8_emit8(v, m, (int)k, row, (int)t8, vg, qs, d);
 }
 
+// RMSNorm of the row of `dim` values that a workgroup's threads hold, 8
+// consecutive ones each (vt: this thread has some): y = (x * w) / rms.
+__device__ __forceinline__ void norm8(const float* x, const float* w, int dim, float eps, bool vt, float* s_red,
+                                      float* y) {
+    float ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) ss += x[e] * x[e];
+    ss = sq_wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    float tot = 0.0f;
+    for (int i = 0; i < kBlock / 64; i++) tot += s_red[i];
+    const float rms = sqrtf(tot / (float)dim + eps);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = vt ? (x[e] * w[e]) / rms : 0.0f;
+}
+__device__ __forceinline__ void load8(const float* p, float* v) {
+    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void store8(float* p, const float* v) {
+    *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+
+// Token rows of a prompt and the first layer's norm of them in one launch:
+// embed_kernel's values (stored to out) through rmsnorm_rows_kernel's vector
+// path, 8 elements per thread (one 8-byte load of payload each; with one byte
+// per load and a launch of their own the rows took 6.7 us for 32 tokens).
+// dim is a multiple of 32, at most 8 * kBlock.
+__global__ __launch_bounds__(kBlock) void embed_norm_kernel(MatView table, const uint32_t* tokens, int dim,
+                                                            float* __restrict__ out, const float* __restrict__ w,
+                                                            float eps, int8_t* __restrict__ act_q,
+                                                            uint16_t* __restrict__ act_d, uint32_t* id_error) {
+    __shared__ float s_red[kBlock / 64];
+    const int r = blockIdx.x, t = threadIdx.x, KB = dim >> 5;
+    const bool vt = 8 * t < dim;
+    float x[8] = {}, wv[8] = {}, y[8];
+    if (vt) load8(w + 8 * t, wv);
+    uint32_t tok = tokens[r];
+    if (tok >= (uint32_t)table.rows) {  // see embed_kernel
+        if (t == 0) *id_error = 1u;
+        tok = table.rows - 1;
+    }
+    if (vt) {
+        const float sc = sq_f16_to_f32(table.scale[(size_t)tok * KB + (t >> 2)]);
+        if (table.wtype == WT_Q8_0) {
+            const uint2 q = *(const uint2*)((const int8_t*)table.qs + (size_t)tok * dim + 8 * t);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                x[e] = sc * sq_sbyte_f((int)q.x, e);
+                x[e + 4] = sc * sq_sbyte_f((int)q.y, e);
+            }
+        } else {  // Q4_0: eight low (elements 0-15 of the block) or high nibbles
+            const uint2 q = *(const uint2*)((const uint8_t*)table.qs + (size_t)tok * (dim / 2) + (t >> 2) * 16 + 8 * (t & 1));
+            const int sh = t & 2 ? 4 : 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                x[e] = sc * (float)((int)((q.x >> (8 * e + sh)) & 15u) - 8);
+                x[e + 4] = sc * (float)((int)((q.y >> (8 * e + sh)) & 15u) - 8);
+            }
+        }
+        store8(out + (size_t)r * dim + 8 * t, x);
+    }
+    norm8(x, wv, dim, eps, vt, s_red, y);
+    q8_emit8(y, gridDim.x, dim, r, t, vt, act_q, act_d);
+}
+
+// The K-split partials of a product summed into the hidden rows (as
+// split_sum4_kernel sums them) and the norm that follows, with its Q8_0
+// blocks, in one launch: the rows are read once instead of written and read
+// back, and one launch fewer (2048 rows of 2048: 13.0 + 9.5 us apart).
+__global__ __launch_bounds__(kBlock) void split_sum_norm_kernel(const float* __restrict__ ws, int splits, size_t stride,
+                                                                int dim, float* __restrict__ hidden,
+                                                                const float* __restrict__ w, float eps,
+                                                                int8_t* __restrict__ act_q,
+                                                                uint16_t* __restrict__ act_d) {
+    __shared__ float s_red[kBlock / 64];
+    const int r = blockIdx.x, t = threadIdx.x;
+    const bool vt = 8 * t < dim;
+    const size_t o = (size_t)r * dim + 8 * t;
+    float x[8] = {}, wv[8] = {}, y[8];
+    if (vt) {
+        float h[8], v[8] = {};
+        load8(hidden + o, h);
+        load8(w + 8 * t, wv);
+        for (int z = 0; z < splits; z++) {
+            float p[8];
+            load8(ws + z * stride + o, p);
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] += p[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = h[e] + v[e];
+        store8(hidden + o, x);
+    }
+    norm8(x, wv, dim, eps, vt, s_red, y);
+    q8_emit8(y, gridDim.x, dim, r, t, vt, act_q, act_d);
+}
+
+// rms_norm over rows (src/ops/rms_norm.rs:13-43); when act_q is non-null the
+// normed row is also quantized to Q8_0 (quantize_row_q8_0, dot_prod.rs:21-31).
 // Rows whose width is a multiple of 8 (of 32 when quantized) and at most
 // 8 * kBlock take the vector path: thread t holds elements 8t..8t+7 (16-byte
 // loads; the lane quad of a 32-element block shares its maximum).  Other
@@ -135,25 +251,14 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(const float* x, co
         (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0) {
         const int t8 = 8 * threadIdx.x;
         const bool vt = t8 < dim;
-        float xv[8] = {}, wv[8] = {};
+        float xv[8] = {}, wv[8] = {}, y[8];
         if (vt) {
-            const float4 a = *(const float4*)(xr + t8), b = *(const float4*)(xr + t8 + 4);
-            const float4 c = *(const float4*)(w + t8), d = *(const float4*)(w + t8 + 4);
-            xv[0] = a.x; xv[1] = a.y; xv[2] = a.z; xv[3] = a.w; xv[4] = b.x; xv[5] = b.y; xv[6] = b.z; xv[7] = b.w;
-            wv[0] = c.x; wv[1] = c.y; wv[2] = c.z; wv[3] = c.w; wv[4] = d.x; wv[5] = d.y; wv[6] = d.z; wv[7] = d.w;
+            load8(xr + t8, xv);
+            load8(w + t8, wv);
         }
-        float ss = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) ss += xv[e] * xv[e];
-        const float rms = row_rms(ss);
-        float y[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) y[e] = vt ? (xv[e] * wv[e]) / rms : 0.0f;
-        if (vt && out) {
-            *(float4*)(out + (size_t)r * dim + t8) = make_float4(y[0], y[1], y[2], y[3]);
-            *(float4*)(out + (size_t)r * dim + t8 + 4) = make_float4(y[4], y[5], y[6], y[7]);
-        }
-        if (act_q) q8_emit8(y, ((size_t)r * dim + t8) / 8, vt, act_q, act_d);
+        norm8(xv, wv, dim, eps, vt, s_red, y);
+        if (vt && out) store8(out + (size_t)r * dim + t8, y);
+        if (act_q) q8_emit8(y, gridDim.x, dim, r, threadIdx.x, vt, act_q, act_d);
         return;
     }
     const bool cached = dim <= NC * kBlock;
@@ -184,8 +289,9 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(const float* x, co
             float scale = sq_q8_scale(amax);
             float inv = sq_q8_inv(scale);
             if (vi) {
-                act_q[(size_t)r * dim + i] = sq_q8_quant(y, inv);
-                if ((i & 31) == 0) act_d[((size_t)r * dim + i) >> 5] = sq_f32_to_f16(scale);
+                act_q[frag_q8(gridDim.x, dim, r, i >> 5) + (size_t)((i >> 4) & 1) * 16 * frag_tile_rows(gridDim.x, r) +
+                      (i & 15)] = sq_q8_quant(y, inv);
+                if ((i & 31) == 0) act_d[frag_scale(gridDim.x, dim >> 5, r, i >> 5)] = sq_f32_to_f16(scale);
             }
         }
     };
@@ -211,8 +317,11 @@ __global__ __launch_bounds__(kBlock) void silu_mul8_kernel(const float* __restri
     const size_t g = (size_t)blockIdx.x * kBlock + threadIdx.x;
     const bool vg = g < n8;
     float v[8] = {};
+    int row = 0;
+    size_t t8 = 0;
     if (vg) {
-        const size_t i = 8 * g, m = i / ffn, j = i % ffn;
+        row_col(g, n8, ffn / 8, row, t8);
+        const size_t m = row, j = 8 * t8;
         const float4* G = (const float4*)(gu + m * 2 * ffn + j);
         const float4* U = (const float4*)(gu + m * 2 * ffn + ffn + j);
         const float4 g0 = G[0], g1 = G[1], u0 = U[0], u1 = U[1];
@@ -228,7 +337,7 @@ __global__ __launch_bounds__(kBlock) void silu_mul8_kernel(const float* __restri
             ((float4*)out)[2 * g + 1] = make_float4(v[4], v[5], v[6], v[7]);
         }
     }
-    if (act_q) q8_emit8(v, g, vg, act_q, act_d);
+    if (act_q) q8_emit8(v, (int)(8 * n8 / ffn), ffn, row, (int)t8, vg, act_q, act_d);
 }
 
 // Split payload/scale <-> GGUF 34-byte Q8_0 blocks (tensor.rs:10-15).
@@ -322,8 +431,10 @@ __global__ __launch_bounds__(kBlock) void silu_mul_kernel(const float* gu, int f
         float scale = sq_q8_scale(amax);
         float inv = sq_q8_inv(scale);
         if (vi) {
-            act_q[i] = sq_q8_quant(f, inv);
-            if ((i & 31) == 0) act_d[i >> 5] = sq_f32_to_f16(scale);
+            const int rows = (int)(n / ffn), row = (int)(i / ffn), c = (int)(i % ffn);
+            act_q[frag_q8(rows, ffn, row, c >> 5) + (size_t)((c >> 4) & 1) * 16 * frag_tile_rows(rows, row) + (c & 15)] =
+                sq_q8_quant(f, inv);
+            if ((c & 31) == 0) act_d[frag_scale(rows, ffn >> 5, row, c >> 5)] = sq_f32_to_f16(scale);
         }
     }
 }
@@ -572,6 +683,41 @@ int launch_embed(hipStream_t s, const MatView& table, int wtype, const uint32_t*
     return check_launch("embed");
 }
 
+bool norm8_fits(int dim) { return dim > 0 && dim % 32 == 0 && dim <= 8 * kBlock; }
+
+int launch_embed_norm(hipStream_t s, const MatView& table, const uint32_t* tokens, int n_tokens, int dim, float* out,
+                      const float* w, float eps, int8_t* act_q, uint16_t* act_d, uint32_t* id_error) {
+    if (!id_error) return set_error(SQ_ERR_ARG, "embed: no error word");
+    hipLaunchKernelGGL(embed_norm_kernel, dim3(n_tokens), dim3(kBlock), 0, s, table, tokens, dim, out, w, eps, act_q,
+                       act_d, id_error);
+    return check_launch("embed_norm");
+}
+
+int launch_split_sum_norm(hipStream_t s, const float* ws, int splits, size_t stride, int m, int dim, float* hidden,
+                          const NormThen& nt) {
+    hipLaunchKernelGGL(split_sum_norm_kernel, dim3(m), dim3(kBlock), 0, s, ws, splits, stride, dim, hidden, nt.w, nt.eps,
+                       nt.act_q, nt.act_d);
+    return check_launch("split_sum_norm");
+}
+
+// What ctx_reset clears, in one launch: the position, the history length and
+// the error words; the epoch moves past every tag an abandoned step may have
+// written.
+__global__ void reset_kernel(int* pos, int* n_hist, uint32_t* id_error, unsigned* epoch, unsigned advance, int* error) {
+    *pos = 0;
+    *n_hist = 0;
+    *id_error = 0;
+    if (epoch) {
+        *epoch += advance;
+        *error = 0;
+    }
+}
+
+int launch_reset(hipStream_t s, int* pos, int* n_hist, uint32_t* id_error, unsigned* epoch, unsigned advance, int* error) {
+    hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(1), 0, s, pos, n_hist, id_error, epoch, advance, error);
+    return check_launch("reset");
+}
+
 int launch_rmsnorm_rows(hipStream_t s, const float* x, const float* w, int rows, int dim, float eps,
                         float* out, int8_t* act_q, uint16_t* act_d) {
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(rows), dim3(kBlock), 0, s, x, w, dim, eps, out, act_q,
@@ -579,13 +725,47 @@ int launch_rmsnorm_rows(hipStream_t s, const float* x, const float* w, int rows,
     return check_launch("rmsnorm_rows");
 }
 
-int launch_quantize_rows(hipStream_t s, const float* x, size_t n, int8_t* qs, uint16_t* d) {
-    if (n % 32 == 0 && ((uintptr_t)x & 15) == 0) {
-        hipLaunchKernelGGL(quantize8_kernel, dim3(grid_for(n / 8, kBlock)), dim3(kBlock), 0, s, x, n / 8, qs, d);
+int launch_quantize_rows(hipStream_t s, const float* x, size_t m, size_t k, int8_t* qs, uint16_t* d) {
+    const size_t n = m * k;
+    if (((uintptr_t)x & 15) == 0) {
+        hipLaunchKernelGGL(quantize8_kernel, dim3(grid_for(n / 8, kBlock)), dim3(kBlock), 0, s, x, (int)m, k, qs, d);
         return check_launch("quantize");
     }
-    hipLaunchKernelGGL(quantize_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s, x, n, qs, d);
+    hipLaunchKernelGGL(quantize_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s, x, (int)m, k, qs, d);
     return check_launch("quantize");
+}
+
+// The fragment-order copy of a matrix of row-order blocks (rows x k/32):
+// thread per (row, block).  Q4_0 nibbles change from q to q - 8 in two's
+// complement (q ^ 8), so that a nibble in the high half of a byte is 16 (q - 8)
+// as a signed byte.
+__global__ __launch_bounds__(kBlock) void frag_copy_kernel(MatView w, uint8_t* __restrict__ fq,
+                                                           uint16_t* __restrict__ fs) {
+    const int KB = w.k >> 5;
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x, n = (size_t)w.rows * KB;
+    if (i >= n) return;
+    // consecutive threads take consecutive rows of a tile: the stores are whole pieces
+    const size_t tile = i / ((size_t)32 * KB);
+    const int rt = frag_tile_rows(w.rows, (int)(32 * tile)), j = (int)(i - tile * 32 * KB);
+    const int row = (int)(32 * tile) + j % rt, kb = j / rt;
+    if (w.wtype == WT_Q8_0) {
+        const sq_v4i* src = (const sq_v4i*)((const int8_t*)w.qs + (size_t)row * w.k + kb * 32);
+        uint8_t* dst = fq + frag_q8(w.rows, w.k, row, kb);
+        *(sq_v4i*)dst = src[0];
+        *(sq_v4i*)(dst + 16 * rt) = src[1];
+    } else {
+        sq_v4i v = *(const sq_v4i*)((const uint8_t*)w.qs + (size_t)row * (w.k / 2) + kb * 16);
+        v ^= (int)0x88888888;
+        *(sq_v4i*)(fq + tile * 16 * w.k + ((size_t)kb * rt + (row & 31)) * 16) = v;
+    }
+    fs[frag_scale(w.rows, KB, row, kb)] = w.scale[(size_t)row * KB + kb];
+}
+
+int launch_frag_copy(hipStream_t s, const DevMatrix& w) {
+    const size_t n = (size_t)w.rows * (w.k / 32);
+    hipLaunchKernelGGL(frag_copy_kernel, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, view(w),
+                       (uint8_t*)w.fq, w.fs);
+    return check_launch("frag_copy");
 }
 
 int launch_pack_q8_blocks(hipStream_t s, const int8_t* qs, const uint16_t* d, size_t nblocks,

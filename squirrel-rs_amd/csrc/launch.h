@@ -80,7 +80,7 @@ int launch_attn_decode_at(hipStream_t s, const float* q, const float* k, const f
                           int n_kv_heads, int head_dim, float* ws, float* out);
 // Prefill: m query rows at positions pos0 .. pos0+m-1 against keys 0..pos0+m-1.
 // Writes the rows to out and/or, when act_q is non-null, their Q8_0 blocks
-// ([m][n_heads*64] and [m][n_heads*2]: what launch_quantize_rows makes of
+// (of m rows of n_heads*64: what launch_quantize_rows makes of
 // out, bit for bit); either may be null.
 // kv_split: attn_split_words(max_keys, n_kv_heads) words of workspace, into
 // which the layer's K and V rows are split (f16 halves) before the
@@ -95,12 +95,36 @@ int launch_sdpa_generic(hipStream_t s, const float* q, const float* k, const flo
                         int seq_q, int seq_k, int n_heads, int n_kv_heads, int head_dim);
 
 // ---- row kernels (k_misc.hip) -------------------------------------------
+// Quantized rows (act_q / act_d, qs / d) are written in fragment order
+// (sq_common.h), which for one row is row order.
 // An id past the table sets *id_error (the row read is clamped in bounds).
 int launch_embed(hipStream_t s, const MatView& table, int wtype, const uint32_t* tokens,
                  int n_tokens, int dim, float* out, uint32_t* id_error);
 int launch_rmsnorm_rows(hipStream_t s, const float* x, const float* w, int rows, int dim,
                         float eps, float* out, int8_t* act_q, uint16_t* act_d);
-int launch_quantize_rows(hipStream_t s, const float* x, size_t n, int8_t* qs, uint16_t* d);
+// The RMSNorm and quantization of a product's output rows that follow it.
+struct NormThen {
+    const float* w;
+    float eps;
+    int8_t* act_q;
+    uint16_t* act_d;
+};
+// Widths the fused norm kernels take.
+bool norm8_fits(int dim);
+// launch_embed and launch_rmsnorm_rows of its rows in one launch (Q8_0 and Q4_0
+// tables, norm8_fits(dim)).
+int launch_embed_norm(hipStream_t s, const MatView& table, const uint32_t* tokens, int n_tokens, int dim, float* out,
+                      const float* w, float eps, int8_t* act_q, uint16_t* act_d, uint32_t* id_error);
+// hidden[m][dim] += the K-split partials in ws, then their norm
+// (norm8_fits(dim); ws, stride and hidden 16-byte aligned).
+int launch_split_sum_norm(hipStream_t s, const float* ws, int splits, size_t stride, int m, int dim, float* hidden,
+                          const NormThen& nt);
+// Clears the position, the history length and the error words; *epoch (null:
+// no persistent step) grows by `advance`.
+int launch_reset(hipStream_t s, int* pos, int* n_hist, uint32_t* id_error, unsigned* epoch, unsigned advance, int* error);
+int launch_quantize_rows(hipStream_t s, const float* x, size_t m, size_t k, int8_t* qs, uint16_t* d);
+// Fills w.fq and w.fs from w.qs and w.scale.
+int launch_frag_copy(hipStream_t s, const DevMatrix& w);
 int launch_pack_q8_blocks(hipStream_t s, const int8_t* qs, const uint16_t* d, size_t nblocks,
                           void* gguf_blocks);
 int launch_unpack_q8_blocks(hipStream_t s, const void* gguf_blocks, size_t nblocks, int8_t* qs,
@@ -145,8 +169,11 @@ int launch_log_softmax_rows(hipStream_t s, const float* logits, size_t stride, i
                             double* out, uint32_t* id_error, void* ws);
 
 // ---- prefill matmul (k_gemm.hip) ----------------------------------------
-// out[m, rows] (+)= in[m, k] @ W.  a8: activations given as Q8_0 (aq/ad,
-// [m][k] / [m][k/32]); otherwise f32 activations x [m][k].
+// out[m, rows] (+)= in[m, k] @ W.  a8: activations given as Q8_0 in fragment
+// order (aq / ad, m rows of k); otherwise f32 activations x [m][k].
+// then (integer path, accumulating into rows of ldo = the matrix's rows): the
+// norm of the output rows that follows, in the launch that sums a K split where
+// there is one.
 // ws: room for ws_floats floats of partial tiles, for a K split of the
 // integer path when the output has few tiles (null: no split).
 constexpr size_t kGemmSplitFloats = (size_t)4 << 20;
@@ -156,19 +183,19 @@ constexpr size_t kPrefillSplitFloats = (size_t)16 << 20;
 // Integer matmul launches on the matrix cores since the last reset: out[0]
 // all, [1] with a K split, [2] on 128 x 128 tiles, [3] the largest split.
 void gemm_counters(bool reset, uint64_t* out);
-int launch_gemm(hipStream_t s, const MatView& w, int wtype, bool a8, const int8_t* aq,
-                const uint16_t* ad, const float* x, int m, float* out, int ldo, bool accumulate,
-                float* ws = nullptr, size_t ws_floats = 0);
+int launch_gemm(hipStream_t s, const DevMatrix& w, bool a8, const int8_t* aq, const uint16_t* ad,
+                const float* x, int m, float* out, int ldo, bool accumulate,
+                float* ws = nullptr, size_t ws_floats = 0, const NormThen* then = nullptr);
 // The FFN gate/up projection (w: [gate | up], 2 * ffn rows) of m prompt rows
-// given as Q8_0, with silu(gate) * up written as Q8_0 blocks (act_q [m][ffn],
-// act_d [m][ffn / 32]) in the same launch: what launch_gemm followed by
+// given as Q8_0, with silu(gate) * up written as Q8_0 blocks (act_q / act_d, m
+// rows of ffn) in the same launch: what launch_gemm followed by
 // launch_silu_mul_rows writes, bit for bit.  act_q/act_d must not overlap
-// aq/ad (every workgroup reads every row).  ws_floats: the workspace size
+// aq/ad (every workgroup reads every row).  ws, ws_floats: the workspace
 // launch_gemm would be given (it picks the same tiling).  Returns -1
 // (nothing launched) where the fused form does not apply (small grids,
 // K-split tilings, pinned tilings).
-int launch_gateup_silu(hipStream_t s, const MatView& w, int wtype, const int8_t* aq, const uint16_t* ad, int m,
-                       int8_t* act_q, uint16_t* act_d, size_t ws_floats = 0);
+int launch_gateup_silu(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint16_t* ad, int m,
+                       int8_t* act_q, uint16_t* act_d, float* ws = nullptr, size_t ws_floats = 0);
 // The stacked q|k|v projection (w: q_dim + 2 kv_dim rows) of m prompt rows
 // at positions pos0.. given as Q8_0, with RoPE on q and k and the KV-cache
 // append in the same launch (or, on a K-split tiling, in the launch that sums
@@ -176,7 +203,7 @@ int launch_gateup_silu(hipStream_t s, const MatView& w, int wtype, const int8_t*
 // launch_rope_kv_rows writes, bit for bit (q_out [m][q_dim], the caches
 // [position][kv_dim]).  Returns -1 (nothing launched) where the fused form
 // does not apply.
-int launch_qkv_rope(hipStream_t s, const MatView& w, int wtype, const int8_t* aq, const uint16_t* ad, int m,
+int launch_qkv_rope(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint16_t* ad, int m,
                     int q_dim, int kv_dim, int head_dim, int pos0, const float2* rope, float* q_out, float* kcache,
                     float* vcache, float* ws = nullptr, size_t ws_floats = 0);
 

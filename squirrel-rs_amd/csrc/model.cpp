@@ -182,7 +182,7 @@ int read_config(const GGUFFile& f, Config* c) {
 }
 
 int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts, const std::vector<size_t>& rows,
-                   size_t k, DevMatrix* out) {
+                   size_t k, DevMatrix* out, bool frag) {
     size_t total = 0;
     for (size_t r : rows) total += r;
     out->wtype = wtype;
@@ -219,18 +219,25 @@ int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts, const st
         if ((st = dmalloc(&out->scale, h_sc.size()))) return st;
         SQ_HIP_CHECK(hipMemcpy(out->scale, h_sc.data(), h_sc.size() * 2, hipMemcpyHostToDevice));
     }
+    if (frag && wtype != WT_BF16 && total) {
+        if ((st = dmalloc((uint8_t**)&out->fq, h_qs.size() + h_sc.size() * 2))) return st;
+        out->fs = (uint16_t*)((uint8_t*)out->fq + h_qs.size());  // (the payload is a multiple of 16 bytes)
+        if ((st = launch_frag_copy(nullptr, *out))) return st;
+        SQ_HIP_CHECK(hipStreamSynchronize(nullptr));
+    }
     return 0;
 }
 
-int upload_matrix(int wtype, const uint8_t* blocks, size_t rows, size_t k, DevMatrix* out) {
-    return upload_stacked(wtype, {blocks}, {rows}, k, out);
+int upload_matrix(int wtype, const uint8_t* blocks, size_t rows, size_t k, DevMatrix* out, bool frag) {
+    return upload_stacked(wtype, {blocks}, {rows}, k, out, frag);
 }
 
 void free_matrix(DevMatrix* m) {
     if (m->qs) (void)hipFree(m->qs);
     if (m->scale) (void)hipFree(m->scale);
-    m->qs = nullptr;
-    m->scale = nullptr;
+    if (m->fq) (void)hipFree(m->fq);
+    m->qs = m->fq = nullptr;
+    m->scale = m->fs = nullptr;
 }
 
 // ---------------------------------------------------------------- model load
@@ -350,19 +357,19 @@ int model_load_impl(const char* path, sq_model** out, bool upload) {
         Layer& L = m->layers[i];
         const LayerSrc& S = src[i];
         if ((st = up_norm(S.an, &L.attn_norm)) || (st = up_norm(S.fn, &L.ffn_norm)) ||
-            (st = upload_stacked(wtype, {S.wq, S.wk, S.wv}, {QD, KVD, KVD}, D, &L.qkv)) ||
-            (st = upload_matrix(wtype, S.wo, D, QD, &L.o)) ||
-            (st = upload_stacked(wtype, {S.wg, S.wu}, {F, F}, D, &L.gateup)) ||
-            (st = upload_matrix(wtype, S.wd, D, F, &L.down)))
+            (st = upload_stacked(wtype, {S.wq, S.wk, S.wv}, {QD, KVD, KVD}, D, &L.qkv, true)) ||
+            (st = upload_matrix(wtype, S.wo, D, QD, &L.o, true)) ||
+            (st = upload_stacked(wtype, {S.wg, S.wu}, {F, F}, D, &L.gateup, true)) ||
+            (st = upload_matrix(wtype, S.wd, D, F, &L.down, true)))
             return fail(st);
         m->weight_bytes += L.qkv.payload_bytes() + L.qkv.scale_bytes() + L.o.payload_bytes() +
                            L.o.scale_bytes() + L.gateup.payload_bytes() + L.gateup.scale_bytes() +
                            L.down.payload_bytes() + L.down.scale_bytes();
     }
-    if ((st = upload_matrix(wtype, we, V, D, &m->embd)) || (st = up_norm(wn, &m->out_norm))) return fail(st);
+    if ((st = upload_matrix(wtype, we, V, D, &m->embd, false)) || (st = up_norm(wn, &m->out_norm))) return fail(st);
     if (tied) {
         m->head = m->embd;
-    } else if ((st = upload_matrix(wtype, wout, V, D, &m->head))) {
+    } else if ((st = upload_matrix(wtype, wout, V, D, &m->head, false))) {
         return fail(st);
     }
     m->tied = tied;
@@ -574,14 +581,14 @@ int run_decode_step(sq_ctx* c) {
     return c->kernels.back()();
 }
 
-// Final norm + LM head + argmax for the last row (prefill tail).
-int run_head(sq_ctx* c, int advance) {
+// Final norm + LM head + argmax for the last row x (prefill tail).
+int run_head(sq_ctx* c, const float* x, int advance) {
     const sq_model* m = c->m;
     const Config& g = m->cfg;
     GemvArgs h{};
     h.w = view(m->head);
     h.n_rows = g.vocab;
-    h.x = c->hidden;
+    h.x = x;
     h.norm_w = m->out_norm;
     h.eps = g.eps;
     h.out = c->logits;
@@ -637,7 +644,14 @@ int run_prefill(sq_ctx* c, size_t n) {
     };
     if ((st = phase(2))) return st;
     SQ_HIP_CHECK(hipMemcpyAsync(c->d_ids, c->h_pinned, n * 4, hipMemcpyHostToDevice, s));
-    if ((st = launch_embed(s, view(m->embd), m->wtype, c->d_ids, (int)n, D, c->p_hidden, c->d_id_error))) return st;
+    // the token rows and, on the integer path, the first layer's norm of them
+    MatView table = view(m->embd);
+    table.wtype = m->wtype;
+    const bool fused_embed = a8 && norm8_fits(D) && !m->layers.empty();
+    if ((st = fused_embed ? launch_embed_norm(s, table, c->d_ids, (int)n, D, c->p_hidden, m->layers[0].attn_norm, g.eps,
+                                              c->p_aq, c->p_ad, c->d_id_error)
+                          : launch_embed(s, table, m->wtype, c->d_ids, (int)n, D, c->p_hidden, c->d_id_error)))
+        return st;
     const int pos0 = (int)c->seq_len;
     const int N = (int)n;
     const size_t kv_layer = c->max_pos * (size_t)KVD;
@@ -645,18 +659,23 @@ int run_prefill(sq_ctx* c, size_t n) {
         const Layer& L = m->layers[l];
         float* kc = c->kcache + l * kv_layer;
         float* vc = c->vcache + l * kv_layer;
-        if ((st = launch_rmsnorm_rows(s, c->p_hidden, L.attn_norm, N, D, g.eps, a8 ? nullptr : c->p_normed,
-                                      a8 ? c->p_aq : nullptr, c->p_ad)) ||
+        // (on the integer path the norms past the first follow the product
+        // before them, see NormThen)
+        const bool normed = a8 && (l > 0 || fused_embed);
+        if ((!normed && (st = launch_rmsnorm_rows(s, c->p_hidden, L.attn_norm, N, D, g.eps, a8 ? nullptr : c->p_normed,
+                                                  a8 ? c->p_aq : nullptr, c->p_ad))) ||
             (st = tap(l, 0, D)))
             return st;
+        const NormThen ffn_norm{L.ffn_norm, g.eps, c->p_aq, c->p_ad};
+        const NormThen next_norm{l + 1 < g.n_layers ? m->layers[l + 1].attn_norm : nullptr, g.eps, c->p_aq, c->p_ad};
         // the q|k|v projection with RoPE and the KV append in its epilogue
         if ((st = phase(0))) return st;
-        const int fused_qkv = a8 ? launch_qkv_rope(s, view(L.qkv), m->wtype, c->p_aq, c->p_ad, N, QD, KVD, hd, pos0,
+        const int fused_qkv = a8 ? launch_qkv_rope(s, L.qkv, c->p_aq, c->p_ad, N, QD, KVD, hd, pos0,
                                                    c->rope, c->p_q, kc, vc, c->p_split, kPrefillSplitFloats)
                                  : -1;
         if (fused_qkv > 0) return fused_qkv;
         if (fused_qkv != 0) {
-            if ((st = launch_gemm(s, view(L.qkv), m->wtype, a8, c->p_aq, c->p_ad, c->p_normed, N, c->p_qkv,
+            if ((st = launch_gemm(s, L.qkv, a8, c->p_aq, c->p_ad, c->p_normed, N, c->p_qkv,
                                   QD + 2 * KVD, false, c->p_split, kPrefillSplitFloats)) ||
                 (st = phase(2)) ||
                 (st = launch_rope_kv_rows(s, c->p_qkv, QD + 2 * KVD, N, QD, KVD, hd, pos0, c->rope, c->p_q, kc, vc)))
@@ -674,12 +693,11 @@ int run_prefill(sq_ctx* c, size_t n) {
             return st;
         if (a8 && (st = tap(l, 1, QD))) return st;
         if ((st = phase(0)) ||
-            (st = launch_gemm(s, view(L.o), m->wtype, a8, c->p_aq, c->p_ad, c->p_attn, N, c->p_hidden, D, true,
-                              c->p_split, kPrefillSplitFloats)) ||
+            (st = launch_gemm(s, L.o, a8, c->p_aq, c->p_ad, c->p_attn, N, c->p_hidden, D, true,
+                              c->p_split, kPrefillSplitFloats, a8 ? &ffn_norm : nullptr)) ||
             (st = phase(2)))
             return st;
-        if ((st = launch_rmsnorm_rows(s, c->p_hidden, L.ffn_norm, N, D, g.eps, a8 ? nullptr : c->p_normed,
-                                      a8 ? c->p_aq : nullptr, c->p_ad)) ||
+        if ((!a8 && (st = launch_rmsnorm_rows(s, c->p_hidden, L.ffn_norm, N, D, g.eps, c->p_normed, nullptr, c->p_ad))) ||
             (st = tap(l, 2, D)))
             return st;
         // Short prompts: gate/up, SiLU * up and its Q8_0 blocks in one launch.
@@ -694,7 +712,7 @@ int run_prefill(sq_ctx* c, size_t n) {
         if (a8) {
             int8_t* aq2 = (int8_t*)c->p_act;
             uint16_t* ad2 = (uint16_t*)(aq2 + (size_t)N * F);
-            fused = launch_gateup_silu(s, view(L.gateup), m->wtype, c->p_aq, c->p_ad, N, aq2, ad2,
+            fused = launch_gateup_silu(s, L.gateup, c->p_aq, c->p_ad, N, aq2, ad2, c->p_split,
                                        kPrefillSplitFloats);
             if (fused > 0) return fused;
             if (fused == 0) {
@@ -703,7 +721,7 @@ int run_prefill(sq_ctx* c, size_t n) {
             }
         }
         if (fused != 0) {
-            if ((st = launch_gemm(s, view(L.gateup), m->wtype, a8, c->p_aq, c->p_ad, c->p_normed, N, c->p_gu, 2 * F,
+            if ((st = launch_gemm(s, L.gateup, a8, c->p_aq, c->p_ad, c->p_normed, N, c->p_gu, 2 * F,
                                   false, c->p_split, kPrefillSplitFloats)) ||
                 (st = phase(2)) ||
                 (st = launch_silu_mul_rows(s, c->p_gu, F, (size_t)N * F, a8 ? nullptr : c->p_act,
@@ -714,14 +732,12 @@ int run_prefill(sq_ctx* c, size_t n) {
         }
         if ((a8 && (st = tap(l, 3, F, fq, fd)))) return st;
         if ((st = phase(0)) ||
-            (st = launch_gemm(s, view(L.down), m->wtype, a8, fq, fd, c->p_act, N, c->p_hidden, D, true,
-                              c->p_split, kPrefillSplitFloats)) ||
+            (st = launch_gemm(s, L.down, a8, fq, fd, c->p_act, N, c->p_hidden, D, true,
+                              c->p_split, kPrefillSplitFloats, a8 && next_norm.w ? &next_norm : nullptr)) ||
             (st = phase(2)))
             return st;
     }
-    SQ_HIP_CHECK(hipMemcpyAsync(c->hidden, c->p_hidden + (size_t)(N - 1) * D, (size_t)D * 4,
-                                hipMemcpyDeviceToDevice, s));
-    if ((st = run_head(c, N))) return st;
+    if ((st = run_head(c, c->p_hidden + (size_t)(N - 1) * D, N))) return st;
     return phase(3);
 }
 
@@ -836,20 +852,12 @@ int ctx_check(sq_ctx* c) {
 int ctx_reset(sq_ctx* c) {
     SQ_HIP_CHECK(hipStreamSynchronize(c->stream));
     c->seq_len = 0;
-    // every write on the context's own stream, so the next launch there is
-    // ordered after them
-    SQ_HIP_CHECK(hipMemsetAsync(c->d_pos, 0, 4, c->stream));
-    SQ_HIP_CHECK(hipMemsetAsync(c->d_nhist, 0, 4, c->stream));
-    SQ_HIP_CHECK(hipMemsetAsync(c->d_id_error, 0, 4, c->stream));
-    if (c->persist) {
-        unsigned epoch = 0;
-        SQ_HIP_CHECK(hipMemcpyAsync(&epoch, c->s_epoch, 4, hipMemcpyDeviceToHost, c->stream));
-        SQ_HIP_CHECK(hipStreamSynchronize(c->stream));
-        epoch += 2u * (6u * (unsigned)c->m->cfg.n_layers + 2u);
-        c->h_pinned[0] = epoch;
-        SQ_HIP_CHECK(hipMemcpyAsync(c->s_epoch, c->h_pinned, 4, hipMemcpyHostToDevice, c->stream));
-        SQ_HIP_CHECK(hipMemsetAsync(c->s_error, 0, 4, c->stream));
-    }
+    // on the context's own stream, so the next launch there is ordered after
+    // it (three fills, an epoch copy there and back and their waits took 60 us)
+    const unsigned advance = 2u * (6u * (unsigned)c->m->cfg.n_layers + 2u);
+    if (int st = launch_reset(c->stream, c->d_pos, c->d_nhist, c->d_id_error, c->persist ? c->s_epoch : nullptr, advance,
+                              c->s_error))
+        return st;
     SQ_HIP_CHECK(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -1103,10 +1111,24 @@ int ctx_read_taps(sq_ctx* c, void* blocks, size_t n_blocks) {
     SQ_HIP_CHECK(hipMemcpy(qs.data() + body, c->head_qs, D, hipMemcpyDeviceToHost));
     SQ_HIP_CHECK(hipMemcpy(d.data() + body / 32, c->head_d, D / 16, hipMemcpyDeviceToHost));
     uint8_t* out = (uint8_t*)blocks;
-    for (size_t b = 0; b < (body + D) / 32; b++) {
-        memcpy(out + 34 * b, &d[b], 2);
-        memcpy(out + 34 * b + 2, qs.data() + 32 * b, 32);
-    }
+    auto put = [&](size_t b, uint16_t scale, const int8_t* lo, const int8_t* hi) {
+        memcpy(out + 34 * b, &scale, 2);
+        memcpy(out + 34 * b + 2, lo, 16);
+        memcpy(out + 34 * b + 18, hi, 16);
+    };
+    // each site's n rows are in fragment order (row order for one row)
+    const size_t width[4] = {D, (size_t)g.n_heads * g.head_dim, D, (size_t)g.ffn};
+    for (int l = 0; l < g.n_layers; l++)
+        for (int j = 0; j < 4; j++) {
+            const size_t off = n * (l * TW + tap_offset(g, j)), k = width[j];
+            for (size_t r = 0; r < n; r++)
+                for (size_t kb = 0; kb < k / 32; kb++) {
+                    const int8_t* lo = qs.data() + off + frag_q8((int)n, (int)k, (int)r, (int)kb);
+                    put((off + r * k) / 32 + kb, d[off / 32 + frag_scale((int)n, (int)(k / 32), (int)r, (int)kb)], lo,
+                        lo + 16 * frag_tile_rows((int)n, (int)r));
+                }
+        }
+    for (size_t b = body / 32; b < (body + D) / 32; b++) put(b, d[b], qs.data() + 32 * b, qs.data() + 32 * b + 16);
     return 0;
 }
 

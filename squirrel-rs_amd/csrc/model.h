@@ -26,11 +26,12 @@ int read_config(const GGUFFile& f, Config* cfg);
 void rope_inv_freq(int head_dim, float base, float factor, float low, float high, float orig_ctx,
                    float* out);
 
-// Upload `rows` rows of GGUF blocks into the device layout (DevMatrix).
-int upload_matrix(int wtype, const uint8_t* blocks, size_t rows, size_t k, DevMatrix* out);
+// Upload `rows` rows of GGUF blocks into the device layout (DevMatrix), with
+// frag also in fragment order (quantized types).
+int upload_matrix(int wtype, const uint8_t* blocks, size_t rows, size_t k, DevMatrix* out, bool frag);
 // Upload several GGUF matrices with equal k as one stacked device matrix.
 int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts,
-                   const std::vector<size_t>& rows, size_t k, DevMatrix* out);
+                   const std::vector<size_t>& rows, size_t k, DevMatrix* out, bool frag);
 void free_matrix(DevMatrix* m);
 
 struct Layer {

@@ -82,7 +82,7 @@ extern "C" int sq_linear_noalloc(const float* d_in, size_t m, size_t k, const sq
     int8_t* aq = (int8_t*)base;
     uint16_t* ad = (uint16_t*)(base + kOffD);
     float* ws = (float*)(base + kOffWs);
-    if ((st = launch_quantize_rows(nullptr, d_in, m * k, aq, ad))) return st;
+    if ((st = launch_quantize_rows(nullptr, d_in, m, k, aq, ad))) return st;
     if (m == 1 && k / 32 <= 256) {
         GemvArgs a{};
         a.w = view(w->m);
@@ -93,7 +93,7 @@ extern "C" int sq_linear_noalloc(const float* d_in, size_t m, size_t k, const sq
         a.out = d_out;
         st = launch_gemv(nullptr, PRO_Q8, EPI_STORE, true, a, nullptr);
     } else {
-        st = launch_gemm(nullptr, view(w->m), w->m.wtype, true, aq, ad, d_in, (int)m, d_out, w->m.rows, false, ws,
+        st = launch_gemm(nullptr, w->m, true, aq, ad, d_in, (int)m, d_out, w->m.rows, false, ws,
                          kGemmSplitFloats);
     }
     if (st) return st;

@@ -45,12 +45,17 @@ constexpr const char* kA32Disabled =
 //          high nibble = element j+16, value (q-8)*scale)
 //   BF16: qs  bf16  [rows][k]        scale unused
 // Bytes per weight are unchanged (1.0625 / 0.5625 / 2).
+//
+// Matrices that the matrix-core kernels multiply have a second copy in
+// fragment order (below): fq and fs, one allocation.
 struct DevMatrix {
     int wtype = 0;
     int rows = 0;
     int k = 0;
     void* qs = nullptr;
     uint16_t* scale = nullptr;
+    void* fq = nullptr;      // Q8_0: int8; Q4_0: packed nibbles of q - 8
+    uint16_t* fs = nullptr;  // (inside fq's allocation)
     size_t payload_bytes() const;
     size_t scale_bytes() const;
 };
@@ -64,6 +69,32 @@ struct MatView {
     int wtype;
     int pad = 0;  // the struct's tail, zero rather than whatever the stack held
 };
+
+// Fragment order of a matrix of quantized rows (activations of more than one
+// row, weights): rows in tiles of 32, and within a tile, block after block,
+// what a wavefront's matrix operand of that block is: the first 16 bytes of
+// each of the tile's rows, then the second 16 bytes of each.  A 64-lane load of
+// an operand is so 1 KB in one piece, where row order made it 64 pieces of 16
+// bytes.  The last tile has only the rows that remain, so the size is that of
+// row order, and one row alone is in row order.  Q4_0 payload: one 16-byte
+// packed block per row instead of the two halves.
+// Block scales: a tile's blocks in pairs, each row's two f16 next to each
+// other (one dword per lane); an odd last block's scales follow unpaired.
+__host__ __device__ inline int frag_tile_rows(int rows, int row) {  // rows in the tile of `row`
+    const int left = rows - (row & ~31);
+    return left < 32 ? left : 32;
+}
+// bytes of half 0 of block kb of `row` (half 1: 16 * frag_tile_rows further)
+__host__ __device__ inline size_t frag_q8(int rows, int k, int row, int kb) {
+    return (size_t)(row >> 5) * 32 * k + ((size_t)kb * 2 * frag_tile_rows(rows, row) + (row & 31)) * 16;
+}
+// index of the f16 scale of block kb of `row`
+__host__ __device__ inline size_t frag_scale(int rows, int kblocks, int row, int kb) {
+    const size_t base = (size_t)(row >> 5) * 32 * kblocks;
+    const int rt = frag_tile_rows(rows, row), r = row & 31;
+    if (kb == kblocks - 1 && (kb & 1) == 0) return base + (size_t)kb * rt + r;
+    return base + ((size_t)(kb >> 1) * rt + r) * 2 + (kb & 1);
+}
 
 inline MatView view(const DevMatrix& m) { return MatView{m.qs, m.scale, m.rows, m.k, m.wtype}; }
 

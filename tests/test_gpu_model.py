@@ -697,6 +697,18 @@ def test_short_prompt_fused_epilogues_bit_exact(model_dir, wtype, monkeypatch):
 
 
 @FULL
+@pytest.mark.parametrize("wtype", ["Q8_0", "Q4_0"])
+@pytest.mark.parametrize("n_prompt", [33, 70, 131, 301, 640])
+def test_full_width_prompt_lengths(model_dir, wtype, n_prompt):
+    """1B widths (2 layers), prompts between the few-rows kernel and the long
+    ones: ragged row tiles, the 64-row shapes, K splits summed with the
+    residual and the following norm, the fused epilogues of both weight
+    types; phase-locked against the oracle."""
+    check_full(full_model(model_dir, wtype, n_layers=2), full_seq(n_prompt, 1, 8), f"1B-wide prompt {n_prompt} {wtype}",
+               max_pos=n_prompt + 8)
+
+
+@FULL
 def test_full_width_long_context_decode(model_dir):
     """1B widths (2 layers), the long-context workload's whole length: a
     4096-token prefill, then all 127 decode steps (positions 4096..4222).  On

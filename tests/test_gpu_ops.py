@@ -248,6 +248,30 @@ def test_matmul_rows_kernel_matches_oracle(wtype, m, k, n, pin, monkeypatch):
     assert np.all(err <= 4e-6 * term_mag(x[rows], wf) + 1e-6), float(err.max())
 
 
+@pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("pin", [None, "64", "128x64", "128"])
+@pytest.mark.parametrize("m,k,n", [
+    (33, 32, 1), (63, 96, 33), (65, 160, 100), (97, 224, 129), (128, 64, 64), (131, 2048, 300), (257, 288, 65),
+    (2, 4128, 40),
+])
+def test_matmul_fragment_order_edges(wtype, pin, m, k, n, monkeypatch):
+    """Operands in fragment order on every tile shape: last tiles of 1 to 31
+    rows and columns, one block of K, odd block counts (an unpaired last
+    scale), K that is not whole groups of four blocks, K splits with a short
+    last part; every output within 4e-6 of its sum of |terms| of the oracle
+    (matmul.rs:133-171), as in the tests of the other shapes."""
+    if pin:
+        monkeypatch.setenv("SQUIRREL_GEMM_TILE", pin)
+    w, _ = quant_weights(wtype, n, k, seed=7 + m)
+    x = (rng(m + k).standard_normal((m, k)) * 1.5).astype(np.float32)
+    out = DeviceArray((m, n))
+    ops.linear(DeviceArray.from_numpy(x), ops.Weight(wtype, w, n, k), out)
+    got = out.numpy().astype(np.float64)
+    want = O.linear(x, wtype, w, n, O.W8A8)
+    wf = np.stack([O.dequantize(wtype, w[i], k) for i in range(n)])
+    assert np.all(np.abs(got - want) <= 4e-6 * term_mag(x, wf) + 1e-6)
+
+
 def test_matmul_rows_kernel_inf_activation_scale():
     """An activation block of f32::MAX/2 has a Q8_0 scale that overflows
     binary16 to inf (dot_prod.rs:629-654): that row's outputs are +-inf or
