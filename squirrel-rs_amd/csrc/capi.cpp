@@ -310,35 +310,44 @@ int sq_quantize_row_q8_0(const float* d_x, size_t n, void* d_blocks) {
 
 namespace {
 
-// Launches the product of one weight with activations already quantized
-// (aq, ad); ws holds kGemmSplitFloats floats of partial tiles.
-int launch_linear(const float* d_in, size_t m, const sq_weight* w, float* d_out, const int8_t* aq, const uint16_t* ad,
-                  float* ws) {
-    const size_t k = w->m.k;
-    if (m == 1 && (k / 32 <= 256)) {
-        GemvArgs a{};
-        a.w = view(w->m);
-        a.n_rows = w->m.rows;
-        a.aq = aq;
-        a.ad = ad;
-        a.x = d_in;
-        a.out = d_out;
-        return launch_gemv(nullptr, PRO_Q8, EPI_STORE, true, a, nullptr);
-    }
-    return launch_gemm(nullptr, w->m, true, aq, ad, d_in, (int)m, d_out, w->m.rows, false, ws,
-                       kGemmSplitFloats);
-}
-
 // Quantizes the m rows once (linear.rs:117-127), multiplies them with each
-// weight and waits once for all of it.
+// weight and waits once for all of it.  One row up to 8192 wide is quantized
+// by the matvec itself.
 int linear_all(const float* d_in, size_t m, size_t k, const sq_weight* const* ws, float* const* d_outs, size_t n) {
     Tmp tq, td, split;
-    int st;
-    if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16))) return st;
-    if (!(m == 1 && (k / 32 <= 256)) && (st = split.alloc(kGemmSplitFloats * sizeof(float)))) return st;
-    st = launch_quantize_rows(nullptr, d_in, m, k, (int8_t*)tq.p, (uint16_t*)td.p);
-    for (size_t i = 0; i < n && !st; i++)
-        st = launch_linear(d_in, m, ws[i], d_outs[i], (const int8_t*)tq.p, (const uint16_t*)td.p, (float*)split.p);
+    int st = 0;
+    const bool matvec = m == 1 && k / 32 <= 256, fused = matvec && ((uintptr_t)d_in & 15) == 0;
+    if (!fused) {
+        if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16)) ||
+            (!matvec && (st = split.alloc(kGemmSplitFloats * sizeof(float)))))
+            return st;
+        st = launch_quantize_rows(nullptr, d_in, m, k, (int8_t*)tq.p, (uint16_t*)td.p);
+    }
+    const int8_t* aq = (const int8_t*)tq.p;
+    const uint16_t* ad = (const uint16_t*)td.p;
+    if (!st && !matvec && n > 1 && n <= (size_t)kSharedMax) {
+        const DevMatrix* mats[kSharedMax];
+        for (size_t i = 0; i < n; i++) mats[i] = &ws[i]->m;
+        st = launch_gemm_shared(nullptr, mats, (int)n, aq, ad, (int)m, d_outs);
+        if (st >= 0) return finish(st);
+        st = 0;
+    }
+    for (size_t i = 0; i < n && !st; i++) {
+        const DevMatrix& w = ws[i]->m;
+        if (matvec) {
+            GemvArgs a{};
+            a.w = view(w);
+            a.n_rows = w.rows;
+            a.aq = aq;
+            a.ad = ad;
+            a.x = d_in;
+            a.out = d_outs[i];
+            st = launch_gemv(nullptr, fused ? PRO_QUANT : PRO_Q8, EPI_STORE, true, a, nullptr);
+        } else {
+            st = launch_gemm(nullptr, w, true, aq, ad, d_in, (int)m, d_outs[i], w.rows, false, (float*)split.p,
+                             kGemmSplitFloats);
+        }
+    }
     return finish(st);
 }
 

@@ -169,7 +169,19 @@ typedef _Float16 mq_v4h __attribute__((ext_vector_type(4)));
 
 // Matmul epilogues: RW_STORE writes (or adds) the tile; RW_GATEUP and RW_QKV
 // are described with the kernels that take them.
-enum : int { RW_STORE = 0, RW_GATEUP = 1, RW_QKV = 2 };
+enum : int { RW_STORE = 0, RW_GATEUP = 1, RW_QKV = 2, RW_SHARED = 3 };
+struct FragMat {  // a matrix in fragment order
+    const int8_t* q;
+    const uint16_t* s;
+    int rows, k;
+};
+// RW_SHARED (the few-rows kernel): further matrices that take the same input;
+// workgroups from begin[i] on multiply w[i], storing to out[i].
+struct SharedMats {
+    FragMat w[kSharedMax - 1];
+    float* out[kSharedMax - 1];
+    int begin[kSharedMax - 1];
+};
 struct RowsEpi {
     int8_t* act_q;       // RW_GATEUP: FFN activation blocks [m][ffn], scales [m][ffn / 32]
     uint16_t* act_d;
@@ -215,12 +227,6 @@ constexpr float kOutScale = WT == WT_Q4_0 ? 1.0f / 16.0f : 1.0f;
 // n ^ 1, lane l ^ 1) and appends the K and V rows to the cache, as
 // rope_kv_kernel does.  The same operations on the same values as the separate
 // kernels, so the same bits.
-struct FragMat {  // a matrix in fragment order
-    const int8_t* q;
-    const uint16_t* s;
-    int rows, k;
-};
-
 // `base` (the same on every lane) plus a lane's byte offset.  The offset is
 // opaque here, so that the address stays a scalar base and a 32-bit lane offset:
 // folded into the loop-invariant part, every tile's 64-bit address would live in
@@ -575,14 +581,27 @@ template <int WT, int NT, int NB, int EPI>
 __global__ __launch_bounds__(RW_NW * 64) void gemm_rows_kernel(FragMat w, const int8_t* __restrict__ aq,
                                                                const uint16_t* __restrict__ ad, int m_rows,
                                                                float* __restrict__ out, int ldo, int accumulate,
-                                                               int per, int kbs, size_t split_stride, RowsEpi ep) {
+                                                               int per, int kbs, size_t split_stride, RowsEpi ep,
+                                                               SharedMats more) {
     constexpr bool GU = EPI == RW_GATEUP;
+    int bx = blockIdx.x;
+    if constexpr (EPI == RW_SHARED) {
+#pragma unroll
+        for (int i = kSharedMax - 2; i >= 0; i--)
+            if (bx >= more.begin[i]) {
+                w = more.w[i];
+                out = more.out[i];
+                ldo = w.rows;
+                bx -= more.begin[i];
+                break;
+            }
+    }
     static_assert(!GU || NT == 2, "the gate/up epilogue pairs two tiles");
     static_assert(EPI != RW_QKV || NT == 1, "the q|k|v epilogue takes one tile");
     __shared__ float red[RW_NW][NT * 16][64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int K = w.k, KB = K >> 5;
-    const int n0 = blockIdx.x * 32 * NT, m0 = blockIdx.y * 32;
+    const int n0 = bx * 32 * NT, m0 = blockIdx.y * 32;
     const int fr = lane & 31, fh = lane >> 5;
     // the workgroup's blocks [kb_begin, kb_end) (split blockIdx.z), and this
     // wavefront's [kbw, kend): per (a multiple of 2 NB) per wavefront
@@ -594,14 +613,14 @@ __global__ __launch_bounds__(RW_NW * 64) void gemm_rows_kernel(FragMat w, const 
     // Operands in fragment order (sq_common.h): per tile its first byte, its
     // rows and this lane's offsets.  Rows and tiles past the end repeat the last
     // one; their results are not stored.
-    const int ffn = w.rows / 2, j0 = blockIdx.x * 32;  // GU: the FFN block's first column
+    const int ffn = w.rows / 2, j0 = bx * 32;  // GU: the FFN block's first column
     const int8_t* pw[NT];
     const uint16_t* psw[NT];
     int rw[NT];
     uint32_t vw[NT], uw[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        const int tile = GU ? t * (ffn >> 5) + (int)blockIdx.x : min(NT * (int)blockIdx.x + t, (w.rows - 1) >> 5);
+        const int tile = GU ? t * (ffn >> 5) + bx : min(NT * bx + t, (w.rows - 1) >> 5);
         rw[t] = frag_tile_rows(w.rows, 32 * tile);
         pw[t] = w.q + (size_t)tile * (WT == WT_Q8_0 ? 32 : 16) * K;
         psw[t] = w.s + (size_t)tile * 32 * KB;
@@ -698,9 +717,9 @@ __global__ __launch_bounds__(RW_NW * 64) void gemm_rows_kernel(FragMat w, const 
             const float scale = sq_q8_scale(fmaxf(mx, 0.0f)), inv = sq_q8_inv(scale);
             const int mm = m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3), jj = l & 31;
             if (mm < m_rows && j0 + jj < ffn) {
-                ep.act_q[frag_q8(m_rows, ffn, mm, blockIdx.x) + (size_t)(jj >> 4) * 16 * frag_tile_rows(m_rows, mm) +
+                ep.act_q[frag_q8(m_rows, ffn, mm, bx) + (size_t)(jj >> 4) * 16 * frag_tile_rows(m_rows, mm) +
                          (jj & 15)] = sq_q8_quant(v, inv);
-                if (jj == 0) ep.act_d[frag_scale(m_rows, ffn / 32, mm, blockIdx.x)] = sq_f32_to_f16(scale);
+                if (jj == 0) ep.act_d[frag_scale(m_rows, ffn / 32, mm, bx)] = sq_f32_to_f16(scale);
             }
         }
         return;
@@ -839,6 +858,8 @@ int splits_for(const DevMatrix& w, int m, int tiles, int target, float* ws, size
     return splits;
 }
 
+// K per wavefront of the few-rows kernel, kbs blocks in all.
+int rows_per_wave(int kbs, int NB) { return ((kbs + RW_NW - 1) / RW_NW + 2 * NB - 1) / (2 * NB) * (2 * NB); }
 // The few-rows kernel: grid (column tiles of 32 NT, row tiles of 32, K
 // splits), K in blocks of 32 with KB a multiple of RW_NB.  Two column tiles
 // per workgroup where that still gives every CU a workgroup (the FFN gate/up
@@ -851,14 +872,14 @@ int launch_rows(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint1
                 bool acc, int gx, int gy, int splits, int kbs, float* ws, const RowsEpi& ep = RowsEpi{},
                 const NormThen** then = nullptr) {
     constexpr int NB = NT == 1 ? RW_NB : RW_NB / 2;
-    const int per = ((kbs + RW_NW - 1) / RW_NW + 2 * NB - 1) / (2 * NB) * (2 * NB);
+    const int per = rows_per_wave(kbs, NB);
     if (splits == 1) {
         hipLaunchKernelGGL((gemm_rows_kernel<WT, NT, NB, EPI>), dim3(gx, gy), dim3(RW_NW * 64), 0, s, frag(w), aq, ad, m, out,
-                           ldo, acc ? 1 : 0, per, kbs, (size_t)0, ep);
+                           ldo, acc ? 1 : 0, per, kbs, (size_t)0, ep, SharedMats{});
     } else {
         const size_t stride = (size_t)m * w.rows;
         hipLaunchKernelGGL((gemm_rows_kernel<WT, NT, NB, RW_STORE>), dim3(gx, gy, splits), dim3(RW_NW * 64), 0, s, frag(w), aq,
-                           ad, m, ws, w.rows, 0, per, kbs, stride, RowsEpi{});
+                           ad, m, ws, w.rows, 0, per, kbs, stride, RowsEpi{}, SharedMats{});
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return set_error(SQ_ERR_HIP, std::string("gemm launch: ") + hipGetErrorString(e));
         if (const int st = launch_split_sum(s, ws, splits, stride, m, w.rows, out, ldo, acc, then)) return st;
@@ -868,20 +889,54 @@ int launch_rows(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint1
     return 0;
 }
 
+struct RowsPlan {
+    bool two;  // two column tiles per workgroup
+    int gx, gy, splits;
+};
+RowsPlan rows_plan(const DevMatrix& w, int m, bool have_ws, size_t ws_floats) {
+    const int KB = w.k / 32, cus = device_cus();
+    const int gy = (m + 31) / 32, tiles = (w.rows + 31) / 32;
+    RowsPlan p{(tiles + 1) / 2 * gy >= cus, 0, gy, 1};
+    p.gx = p.two ? (tiles + 1) / 2 : tiles;
+    if (have_ws && p.gx * gy < cus) {
+        int splits = min((cus + p.gx * gy - 1) / (p.gx * gy), KB / (RW_NW * 2 * RW_NB));
+        while (splits > 1 && ((size_t)splits * m * w.rows > ws_floats || KB % splits || (KB / splits) % RW_NB))
+            splits--;
+        p.splits = max(splits, 1);
+    }
+    return p;
+}
+
+template <int WT>
+int run_rows_shared(hipStream_t s, const DevMatrix* const* ws, int n, const int8_t* aq, const uint16_t* ad, int m,
+                    float* const* outs) {
+    SharedMats more{};
+    int gx = 0;
+    for (int i = 0; i < n; i++) {
+        if (i > 0) {
+            more.w[i - 1] = frag(*ws[i]);
+            more.out[i - 1] = outs[i];
+            more.begin[i - 1] = gx;
+        }
+        gx += (ws[i]->rows + 31) / 32;
+        count_launch(1, 32);
+    }
+    for (int i = n - 1; i < kSharedMax - 1; i++) more.begin[i] = INT32_MAX;
+    const int KB = ws[0]->k / 32;
+    hipLaunchKernelGGL((gemm_rows_kernel<WT, 1, RW_NB, RW_SHARED>), dim3(gx, (m + 31) / 32), dim3(RW_NW * 64), 0, s,
+                       frag(*ws[0]), aq, ad, m, outs[0], ws[0]->rows, 0, rows_per_wave(KB, RW_NB), KB, (size_t)0,
+                       RowsEpi{}, more);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(SQ_ERR_HIP, std::string("gemm launch: ") + hipGetErrorString(e));
+    return 0;
+}
+
 template <int WT>
 int run_rows(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint16_t* ad, int m, float* out, int ldo,
              bool acc, float* ws, size_t ws_floats, const NormThen** then) {
-    const int KB = w.k / 32, cus = device_cus();
-    const int gy = (m + 31) / 32, tiles = (w.rows + 31) / 32;
-    const bool two = (tiles + 1) / 2 * gy >= cus;
-    const int gx = two ? (tiles + 1) / 2 : tiles;
-    int splits = 1;
-    if (ws != nullptr && gx * gy < cus) {
-        splits = min((cus + gx * gy - 1) / (gx * gy), KB / (RW_NW * 2 * RW_NB));
-        while (splits > 1 && ((size_t)splits * m * w.rows > ws_floats || KB % splits || (KB / splits) % RW_NB))
-            splits--;
-        splits = max(splits, 1);
-    }
+    const RowsPlan p = rows_plan(w, m, ws != nullptr, ws_floats);
+    const bool two = p.two;
+    const int KB = w.k / 32, gx = p.gx, gy = p.gy, splits = p.splits;
     const int kbs = KB / splits;
     count_launch(splits, 32);
     return two ? launch_rows<WT, 2>(s, w, aq, ad, m, out, ldo, acc, gx, gy, splits, kbs, ws, RowsEpi{}, then)
@@ -910,8 +965,8 @@ bool rows_kernel_fits(int m, int k) { return m <= 32 && (k / 32) % RW_NB == 0 &&
 // tiling pinned, shared by the plain path and the fused epilogues so that both
 // fold the same terms:
 //  - matrices of 8192 and more rows whose input would leave an eighth of its
-//    128-row tiles empty: 64-row tiles, unsplit, where those give every CU two
-//    workgroups (a wavefront of 32 x 64 spends 14% more per output than one of
+//    128-row tiles empty: 64-row tiles, unsplit, from one and a half workgroups
+//    per CU on (a wavefront of 32 x 64 spends 14% more per output than one of
 //    64 x 64: 156 against 137 us for 2048 x 16384 x 2048; of 320 rows, 384 in
 //    128-row tiles, 37 against 41);
 //  - 128 x 128 tiles where they give every CU two workgroups;
@@ -929,7 +984,8 @@ struct Tiling {
 Tiling auto_tiling(const DevMatrix& w, int m, float* ws, size_t ws_floats) {
     const int cus = device_cus(), gy = (m + 127) / 128, gy64 = (m + 63) / 64;
     const int g = (w.rows + 127) / 128 * gy, g64 = (w.rows + 63) / 64 * gy64;
-    if (w.rows >= 8192 && 128 * gy * 7 >= 64 * gy64 * 8 && (w.rows + 127) / 128 * gy64 >= 2 * cus) return {SHAPE_64X128, 1};
+    if (w.rows >= 8192 && 128 * gy * 7 >= 64 * gy64 * 8 && 2 * ((w.rows + 127) / 128 * gy64) >= 3 * cus)
+        return {SHAPE_64X128, 1};
     if (m >= 128) {
         if (g >= 2 * cus) return {SHAPE_128, 1};
         if (w.k / 32 >= 64 && ws != nullptr && w.rows < 8192) {
@@ -1060,6 +1116,22 @@ void gemm_counters(bool reset, uint64_t* out) {
         g_tile128x64_launches = 0;
         g_rows_launches = 0;
     }
+}
+
+int launch_gemm_shared(hipStream_t s, const DevMatrix* const* ws, int n, const int8_t* aq, const uint16_t* ad, int m,
+                       float* const* outs) {
+    if (n < 1 || n > kSharedMax || m <= 0) return -1;
+    for (int i = 0; i < n; i++) {
+        const DevMatrix& w = *ws[i];
+        if (w.fq == nullptr || w.wtype != ws[0]->wtype || w.k != ws[0]->k || w.k <= 0 || w.k % 32 != 0 || w.rows <= 0 ||
+            !rows_kernel_fits(m, w.k))
+            return -1;
+        const RowsPlan p = rows_plan(w, m, true, kGemmSplitFloats);
+        if (p.two || p.splits != 1) return -1;
+    }
+    if (ws[0]->wtype == WT_Q8_0) return run_rows_shared<WT_Q8_0>(s, ws, n, aq, ad, m, outs);
+    if (ws[0]->wtype == WT_Q4_0) return run_rows_shared<WT_Q4_0>(s, ws, n, aq, ad, m, outs);
+    return -1;
 }
 
 int launch_gateup_silu(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint16_t* ad, int m, int8_t* act_q,

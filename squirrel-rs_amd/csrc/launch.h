@@ -11,6 +11,8 @@ enum GemvPro : int {
                    // quantized (A8) or kept f32 (A32) in LDS
     PRO_Q8 = 1,    // quantized activation blocks read from global memory
     PRO_F32 = 2,   // f32 activations read from global memory
+    PRO_QUANT = 3, // f32 activations (16-byte aligned), each lane quantizing the
+                   // blocks it multiplies
 };
 enum GemvEpi : int {
     EPI_STORE = 0,   // out[row] = v
@@ -186,6 +188,13 @@ void gemm_counters(bool reset, uint64_t* out);
 int launch_gemm(hipStream_t s, const DevMatrix& w, bool a8, const int8_t* aq, const uint16_t* ad,
                 const float* x, int m, float* out, int ldo, bool accumulate,
                 float* ws = nullptr, size_t ws_floats = 0, const NormThen* then = nullptr);
+// The products of one input with n matrices of equal k in one launch, where
+// the few-rows kernel takes each of them unsplit with a tile per workgroup:
+// what launch_gemm writes for each with the same workspace size, bit for bit.
+// Returns -1 (nothing launched) where that does not apply.
+constexpr int kSharedMax = 4;
+int launch_gemm_shared(hipStream_t s, const DevMatrix* const* ws, int n, const int8_t* aq, const uint16_t* ad, int m,
+                       float* const* outs);
 // The FFN gate/up projection (w: [gate | up], 2 * ffn rows) of m prompt rows
 // given as Q8_0, with silu(gate) * up written as Q8_0 blocks (act_q / act_d, m
 // rows of ffn) in the same launch: what launch_gemm followed by
