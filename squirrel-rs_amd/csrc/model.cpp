@@ -771,8 +771,9 @@ int setup_persistent(sq_ctx* c) {
     }
     const size_t nx = exchange_words(g.dim, g.ffn, g.n_heads, g.n_kv_heads, c->max_tiles, grid);
     if ((st = dmalloc(&c->d_layers, (size_t)g.n_layers)) || (st = dmalloc(&c->s_xchg, nx)) ||
-        (st = dmalloc(&c->s_epoch, 1)) || (st = dmalloc(&c->s_error, 1)))
+        (st = dmalloc(&c->s_epoch, 1)))
         return st;
+    c->s_error = (int*)(c->d_id_error + 1);
     SQ_HIP_CHECK(hipMemcpy(c->d_layers, hl.data(), hl.size() * sizeof(StepLayer), hipMemcpyHostToDevice));
     SQ_HIP_CHECK(hipMemset(c->s_xchg, 0, nx * 8));
     SQ_HIP_CHECK(hipMemset(c->s_epoch, 0, 4));
@@ -836,15 +837,12 @@ int setup_persistent(sq_ctx* c) {
 
 int ctx_check(sq_ctx* c) {
     SQ_HIP_CHECK(hipStreamSynchronize(c->stream));
-    uint32_t id_err = 0;
-    SQ_HIP_CHECK(hipMemcpy(&id_err, c->d_id_error, 4, hipMemcpyDeviceToHost));
-    if (id_err)
+    uint32_t words[2] = {0, 0};  // d_id_error and s_error, in one copy
+    SQ_HIP_CHECK(hipMemcpy(words, c->d_id_error, 8, hipMemcpyDeviceToHost));
+    if (words[0])
         return set_error(SQ_ERR_ARG, "forward: a token id on the device is past the embedding table "
                                      "(embedding.rs:43-44); the context must be reset");
-    if (!c->persist) return 0;
-    int err = 0;
-    SQ_HIP_CHECK(hipMemcpy(&err, c->s_error, 4, hipMemcpyDeviceToHost));
-    if (err)
+    if (c->persist && words[1])
         return set_error(SQ_ERR_HIP, "decode step: a grid barrier wait timed out; the context must be reset");
     return 0;
 }
@@ -899,7 +897,7 @@ int ctx_create(const sq_model* m, size_t max_pos, uint32_t flags, sq_ctx** out) 
         (st = dmalloc(&c->dbg_normed, D)) || (st = dmalloc(&c->last_hidden, D)) || (st = dmalloc(&c->head_qs, D)) ||
         (st = dmalloc(&c->head_d, D / 32)) || (st = dmalloc(&c->d_sids, 2 * (max_pos + 1))) ||
         (st = dmalloc(&c->d_logp, max_pos + 1)) ||
-        (st = dmalloc((uint8_t**)&c->lsm_ws, kScoreRows * (size_t)log_softmax_parts(g.vocab) * kLsmPartBytes)) || (st = dmalloc(&c->d_id_error, 1)))
+        (st = dmalloc((uint8_t**)&c->lsm_ws, kScoreRows * (size_t)log_softmax_parts(g.vocab) * kLsmPartBytes)) || (st = dmalloc(&c->d_id_error, 2)))
         return fail(st);
     he = hipHostMalloc((void**)&c->h_pinned, (max_pos + 16) * sizeof(uint32_t), hipHostMallocDefault);
     if (he != hipSuccess) return fail(set_error(SQ_ERR_HIP, std::string("hipHostMalloc: ") + hipGetErrorString(he)));
@@ -923,7 +921,7 @@ int ctx_create(const sq_model* m, size_t max_pos, uint32_t flags, sq_ctx** out) 
     SQ_HIP_CHECK(hipMemset(c->d_pos, 0, 4));
     SQ_HIP_CHECK(hipMemset(c->d_nhist, 0, 4));
     SQ_HIP_CHECK(hipMemset(c->d_token, 0, 4));
-    SQ_HIP_CHECK(hipMemset(c->d_id_error, 0, 4));
+    SQ_HIP_CHECK(hipMemset(c->d_id_error, 0, 8));
     SQ_HIP_CHECK(hipMemset(c->kcache, 0, (size_t)g.n_layers * max_pos * KVD * 4));
     SQ_HIP_CHECK(hipMemset(c->vcache, 0, (size_t)g.n_layers * max_pos * KVD * 4));
 
@@ -957,7 +955,7 @@ void ctx_destroy(sq_ctx* c) {
     dfree(c->last_hidden); dfree(c->head_qs); dfree(c->head_d);
     dfree(c->p_hidden); dfree(c->p_normed); dfree(c->p_qkv); dfree(c->p_q); dfree(c->p_attn); dfree(c->p_gu);
     dfree(c->p_kvs); dfree(c->p_act); dfree(c->p_aq); dfree(c->p_ad); dfree(c->p_split);
-    dfree(c->d_layers); dfree(c->s_stream); dfree(c->s_xchg); dfree(c->s_epoch); dfree(c->s_error); dfree(c->s_trace);
+    dfree(c->d_layers); dfree(c->s_stream); dfree(c->s_xchg); dfree(c->s_epoch); dfree(c->s_trace);
     dfree(c->d_sids); dfree(c->d_logp); dfree(c->s_rows); dfree(c->lsm_ws); dfree(c->d_id_error);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
     if (c->stream) (void)hipStreamDestroy(c->stream);

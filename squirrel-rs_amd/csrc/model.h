@@ -129,7 +129,7 @@ struct sq_ctx {
     uint8_t* s_stream = nullptr;  // per-CU weight streams
     unsigned long long* s_xchg = nullptr;  // exchange words
     unsigned* s_epoch = nullptr;
-    int* s_error = nullptr;
+    int* s_error = nullptr;  // the word after d_id_error, in its allocation
     unsigned long long* s_trace = nullptr;  // step timeline when enabled
 
     // Set by a kernel that met a token id past the embedding table (the

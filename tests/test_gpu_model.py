@@ -522,10 +522,12 @@ def test_score_rows_at_batch_edges(ppl_gguf, steps):
         want.append(seq_log_softmax_at(f.logits(), int(window[burn + i])))
     assert np.abs(got - np.array(want)).max() < 1e-12
     assert np.array_equal(c.logits(), f.logits()) and c.argmax() == f.argmax()
-    # decoding goes on from the scored window
+    # decoding goes on from the scored window (one context at a time: a
+    # persistent step needs every CU for itself)
     c.forward([7])
+    after = c.logits()
     f.forward([7])
-    assert np.array_equal(c.logits(), f.logits())
+    assert np.array_equal(after, f.logits())
 
 
 def test_perplexity_harness(ppl_gguf):
