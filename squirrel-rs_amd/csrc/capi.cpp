@@ -311,18 +311,15 @@ int sq_quantize_row_q8_0(const float* d_x, size_t n, void* d_blocks) {
 namespace {
 
 // Quantizes the m rows once (linear.rs:117-127), multiplies them with each
-// weight and waits once for all of it.  One row up to 8192 wide is quantized
-// by the matvec itself.
+// weight and waits once for all of it.
 int linear_all(const float* d_in, size_t m, size_t k, const sq_weight* const* ws, float* const* d_outs, size_t n) {
     Tmp tq, td, split;
     int st = 0;
-    const bool matvec = m == 1 && k / 32 <= 256, fused = matvec && ((uintptr_t)d_in & 15) == 0;
-    if (!fused) {
-        if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16)) ||
-            (!matvec && (st = split.alloc(kGemmSplitFloats * sizeof(float)))))
-            return st;
-        st = launch_quantize_rows(nullptr, d_in, m, k, (int8_t*)tq.p, (uint16_t*)td.p);
-    }
+    const bool matvec = m == 1 && k / 32 <= 256;
+    if ((st = tq.alloc(m * k)) || (st = td.alloc(m * k / 16)) ||
+        (!matvec && (st = split.alloc(kGemmSplitFloats * sizeof(float)))))
+        return st;
+    st = launch_quantize_rows(nullptr, d_in, m, k, (int8_t*)tq.p, (uint16_t*)td.p);
     const int8_t* aq = (const int8_t*)tq.p;
     const uint16_t* ad = (const uint16_t*)td.p;
     if (!st && !matvec && n > 1 && n <= (size_t)kSharedMax) {
@@ -342,7 +339,7 @@ int linear_all(const float* d_in, size_t m, size_t k, const sq_weight* const* ws
             a.ad = ad;
             a.x = d_in;
             a.out = d_outs[i];
-            st = launch_gemv(nullptr, fused ? PRO_QUANT : PRO_Q8, EPI_STORE, true, a, nullptr);
+            st = launch_gemv(nullptr, PRO_Q8, EPI_STORE, true, a, nullptr);
         } else {
             st = launch_gemm(nullptr, w, true, aq, ad, d_in, (int)m, d_outs[i], w.rows, false, (float*)split.p,
                              kGemmSplitFloats);

@@ -28,7 +28,6 @@ namespace sq {
 namespace {
 
 constexpr int kPad = 36;  // f32 activation LDS stride per 32-block (bank spread)
-typedef float sq_v4f __attribute__((ext_vector_type(4)));
 
 template <int WT>
 struct WBlk;
@@ -184,16 +183,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvArgs a) {
             ASUM[b] = 0;
         }
     }
-    // PRO_QUANT: this lane's f32 blocks, one at a time for more than one per
-    // lane (the others are requested as they are used)
-    sq_v4f xq[PRO == PRO_QUANT ? 8 : 1];
-    auto load_x = [&](int b) {
-        const int blk = lane + 64 * b;
-        const sq_v4f* p = (const sq_v4f*)(a.x + (size_t)(blk < KB ? blk : 0) * 32);
-#pragma unroll
-        for (int v = 0; v < (PRO == PRO_QUANT ? 8 : 1); v++) xq[v] = p[v];
-    };
-    if constexpr (PRO == PRO_QUANT) load_x(0);
     // The RoPE position, read before the weight stream is requested.
     int qkv_pos = 0;
     if constexpr (EPI == EPI_QKV) qkv_pos = *a.pos;
@@ -283,32 +272,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvArgs a) {
                 for (int v = 0; v < 8; v++) sacc = __builtin_amdgcn_sdot4(AQ[b][v], 0x01010101, sacc, false);
                 ASUM[b] = sacc;
             }
-        }
-    } else if constexpr (PRO == PRO_QUANT) {
-        // quantize_row_q8_0 (dot_prod.rs:21-31) of the lane's own blocks, while
-        // the weight stream is in flight: a launch of its own for it, with
-        // the blocks written and read back, took 2.2 us and the gap after it
-#pragma unroll
-        for (int b = 0; b < NBL; b++) {
-            if (b > 0) load_x(b);
-            float amax = 0.0f;
-#pragma unroll
-            for (int v = 0; v < 8; v++)
-#pragma unroll
-                for (int c = 0; c < 4; c++) amax = fmaxf(amax, fabsf(xq[v][c]));
-            const float scale = sq_q8_scale(amax), inv = sq_q8_inv(scale);
-            const bool vb = lane + 64 * b < KB;
-            int sacc = 0;
-#pragma unroll
-            for (int v = 0; v < 8; v++) {
-                unsigned w = 0;
-#pragma unroll
-                for (int c = 0; c < 4; c++) w |= (unsigned)(uint8_t)sq_q8_quant(xq[v][c], inv) << (8 * c);
-                AQ[b][v] = vb ? (int)w : 0;
-                if constexpr (WT == WT_Q4_0) sacc = __builtin_amdgcn_sdot4(AQ[b][v], 0x01010101, sacc, false);
-            }
-            AS[b] = vb ? sq_f16_to_f32(sq_f32_to_f16(scale)) : 0.0f;
-            ASUM[b] = sacc;
         }
     } else {  // PRO_F32
         for (int i = tid; i < K; i += G::NT) s_x[(i >> 5) * kPad + (i & 31)] = a.x[i];
@@ -563,10 +526,6 @@ int dispatch(hipStream_t s, int pro, int epi, const GemvArgs& a, int* grid_out) 
             if (KB <= 256) return run<WT, A8, 4, 1, 4, PRO_A, EPI_RESID>(s, a, 1 << 30, grid_out);
             break;
         case EPI_STORE:
-            if constexpr (A8) {
-                if (pro == PRO_QUANT && KB <= 64) return run<WT, A8, 1, 2, 4, PRO_QUANT, EPI_STORE>(s, a, 1 << 30, grid_out);
-                if (pro == PRO_QUANT && KB <= 256) return run<WT, A8, 4, 1, 4, PRO_QUANT, EPI_STORE>(s, a, 1 << 30, grid_out);
-            }
             if (pro != PRO_A) break;
             if (KB <= 64) return run<WT, A8, 1, 2, 4, PRO_A, EPI_STORE>(s, a, 1 << 30, grid_out);
             if (KB <= 256) return run<WT, A8, 4, 1, 4, PRO_A, EPI_STORE>(s, a, 1 << 30, grid_out);

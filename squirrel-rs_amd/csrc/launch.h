@@ -11,8 +11,6 @@ enum GemvPro : int {
                    // quantized (A8) or kept f32 (A32) in LDS
     PRO_Q8 = 1,    // quantized activation blocks read from global memory
     PRO_F32 = 2,   // f32 activations read from global memory
-    PRO_QUANT = 3, // f32 activations (16-byte aligned), each lane quantizing the
-                   // blocks it multiplies
 };
 enum GemvEpi : int {
     EPI_STORE = 0,   // out[row] = v

@@ -331,40 +331,6 @@ def test_matmul_subnormal_activation_scales(tile, monkeypatch):
 
 
 @pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0])
-@pytest.mark.parametrize("k", [32, 2048, 2080, 4128, 8192])
-def test_one_row_quantized_in_the_matvec(wtype, k):
-    """One row goes to the matvec as f32 (each lane quantizes its own blocks)
-    when 16-byte aligned, and through the quantizer's launch otherwise: the
-    same bits, for one to four blocks per lane and a part-filled last round;
-    a row with an infinite block scale gives what the two launches give."""
-    n = 37
-    w, _ = quant_weights(wtype, n, k, seed=k)
-    W = ops.Weight(wtype, w, n, k)
-    x = rng(k).standard_normal((1, k)).astype(np.float32)
-    big = np.zeros(k + 4, np.float32)
-
-    def both(x):
-        out, out2 = DeviceArray((1, n)), DeviceArray((1, n))
-        ops.linear(DeviceArray.from_numpy(x), W, out)
-        big[1:k + 1] = x[0]
-        buf = DeviceArray.from_numpy(big)
-
-        class Off:
-            ptr, shape, size = buf.ptr + 4, (1, k), k
-        ops.linear(Off, W, out2)
-        return out.numpy(), out2.numpy()
-
-    a, b = both(x)
-    assert np.array_equal(a, b) and np.all(np.isfinite(a))
-    want = O.linear(x, wtype, w, n, O.W8A8)
-    wf = np.stack([O.dequantize(wtype, w[i], k) for i in range(n)])
-    assert np.all(np.abs(a.astype(np.float64) - want) <= 4e-6 * term_mag(x, wf) + 1e-6)
-    x[0, :32] = np.float32(np.finfo(np.float32).max / 2)
-    a, b = both(x)
-    assert np.array_equal(a, b, equal_nan=True)
-
-
-@pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0])
 @pytest.mark.parametrize("m,k,rows", [(2, 128, (7, 100, 33)), (32, 2048, (2048, 512, 512)), (9, 512, (512, 128)),
                                       (5, 256, (64, 1, 32, 31)), (32, 2048, (8192, 8192)), (3, 96, (40, 50))])
 def test_linear_shared_one_launch_equals_separate(wtype, m, k, rows):
