@@ -568,7 +568,7 @@ int launch_split_sum(hipStream_t s, const float* ws, int splits, size_t stride, 
 // pair partner of column n is column n ^ 1, lane l ^ 1).  The same
 // operations on the same values, so the same bits as the separate kernels.
 constexpr int RW_NW = 8;  // wavefronts per workgroup
-constexpr int RW_NB = 4;  // blocks per load batch with one column tile (two with two)
+constexpr int RW_NB = 4;  // blocks per load batch
 
 template <int NT, int NB>
 struct RwBatch {
@@ -599,7 +599,8 @@ __global__ __launch_bounds__(RW_NW * 64) void gemm_rows_kernel(FragMat w, const 
     static_assert(!GU || NT == 2, "the gate/up epilogue pairs two tiles");
     static_assert(EPI != RW_QKV || NT == 1, "the q|k|v epilogue takes one tile");
     __shared__ float red[RW_NW][NT * 16][64];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int K = w.k, KB = K >> 5;
     const int n0 = bx * 32 * NT, m0 = blockIdx.y * 32;
     const int fr = lane & 31, fh = lane >> 5;
@@ -639,14 +640,16 @@ __global__ __launch_bounds__(RW_NW * 64) void gemm_rows_kernel(FragMat w, const 
         for (int j = 0; j < NB; j++) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
-                B.w[t][j] = *(const sq_v4i*)(pw[t] + (size_t)(kc + j) * ((WT == WT_Q8_0 ? 32 : 16) * rw[t]) + vw[t]);
-            B.a[j] = *(const sq_v4i*)(pa + (size_t)(kc + j) * (32 * ra) + va);
+                B.w[t][j] =
+                    *(const sq_v4i*)lane_at(pw[t] + (size_t)(kc + j) * ((WT == WT_Q8_0 ? 32 : 16) * rw[t]), vw[t]);
+            B.a[j] = *(const sq_v4i*)lane_at(pa + (size_t)(kc + j) * (32 * ra), va);
         }
 #pragma unroll
         for (int j = 0; j < NB; j += 2) {
 #pragma unroll
-            for (int t = 0; t < NT; t++) B.sw[t][j / 2] = *(const uint32_t*)(psw[t] + (size_t)(kc + j) * rw[t] + 2 * uw[t]);
-            B.sa[j / 2] = *(const uint32_t*)(psa + (size_t)(kc + j) * ra + 2 * ua);
+            for (int t = 0; t < NT; t++)
+                B.sw[t][j / 2] = *(const uint32_t*)lane_at(psw[t] + (size_t)(kc + j) * rw[t], 4 * uw[t]);
+            B.sa[j / 2] = *(const uint32_t*)lane_at(psa + (size_t)(kc + j) * ra, 4 * ua);
         }
     };
     m8_v16f acc[NT];
@@ -871,7 +874,7 @@ template <int WT, int NT, int EPI = RW_STORE>
 int launch_rows(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint16_t* ad, int m, float* out, int ldo,
                 bool acc, int gx, int gy, int splits, int kbs, float* ws, const RowsEpi& ep = RowsEpi{},
                 const NormThen** then = nullptr) {
-    constexpr int NB = NT == 1 ? RW_NB : RW_NB / 2;
+    constexpr int NB = RW_NB;
     const int per = rows_per_wave(kbs, NB);
     if (splits == 1) {
         hipLaunchKernelGGL((gemm_rows_kernel<WT, NT, NB, EPI>), dim3(gx, gy), dim3(RW_NW * 64), 0, s, frag(w), aq, ad, m, out,
