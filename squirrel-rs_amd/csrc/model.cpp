@@ -190,15 +190,21 @@ int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts, const st
     out->k = (int)k;
     const size_t kb = k / 32;
     const size_t pay = row_payload_bytes(wtype, k);
-    std::vector<uint8_t> h_qs(total * pay);
-    std::vector<uint16_t> h_sc(wtype == WT_BF16 ? 0 : total * kb);
+    // one allocation: payload, scales, then the fragment-order copies of both,
+    // each on a 256-byte boundary
+    auto up256 = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t q_bytes = total * pay, s_bytes = wtype == WT_BF16 ? 0 : total * kb * 2;
+    const size_t s_off = up256(q_bytes), f_off = s_off + up256(s_bytes);
+    frag = frag && wtype != WT_BF16 && total;
+    std::vector<uint8_t> h(s_off + s_bytes);
+    uint16_t* const h_sc = (uint16_t*)(h.data() + s_off);
     size_t r0 = 0;
     for (size_t p = 0; p < parts.size(); p++) {
         const uint8_t* src = parts[p];
         const size_t grb = gguf_row_bytes(wtype, k);
         for (size_t r = 0; r < rows[p]; r++) {
             const uint8_t* row = src + r * grb;
-            uint8_t* dq = h_qs.data() + (r0 + r) * pay;
+            uint8_t* dq = h.data() + (r0 + r) * pay;
             if (wtype == WT_BF16) {
                 memcpy(dq, row, pay);
                 continue;
@@ -213,17 +219,15 @@ int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts, const st
         r0 += rows[p];
     }
     int st;
-    if ((st = dmalloc((uint8_t**)&out->qs, h_qs.size()))) return st;
-    SQ_HIP_CHECK(hipMemcpy(out->qs, h_qs.data(), h_qs.size(), hipMemcpyHostToDevice));
-    if (!h_sc.empty()) {
-        if ((st = dmalloc(&out->scale, h_sc.size()))) return st;
-        SQ_HIP_CHECK(hipMemcpy(out->scale, h_sc.data(), h_sc.size() * 2, hipMemcpyHostToDevice));
-    }
-    if (frag && wtype != WT_BF16 && total) {
-        if ((st = dmalloc((uint8_t**)&out->fq, h_qs.size() + h_sc.size() * 2))) return st;
-        out->fs = (uint16_t*)((uint8_t*)out->fq + h_qs.size());  // (the payload is a multiple of 16 bytes)
+    if ((st = dmalloc((uint8_t**)&out->qs, frag ? f_off + up256(q_bytes) + s_bytes : h.size()))) return st;
+    if (!h.empty()) SQ_HIP_CHECK(hipMemcpy(out->qs, h.data(), h.size(), hipMemcpyHostToDevice));
+    if (s_bytes) out->scale = (uint16_t*)((uint8_t*)out->qs + s_off);
+    if (frag) {
+        out->fq = (uint8_t*)out->qs + f_off;
+        out->fs = (uint16_t*)((uint8_t*)out->fq + up256(q_bytes));
+        // on the null stream, as the operators' launches are; a context's own
+        // stream starts after the device has been waited for
         if ((st = launch_frag_copy(nullptr, *out))) return st;
-        SQ_HIP_CHECK(hipStreamSynchronize(nullptr));
     }
     return 0;
 }
@@ -233,9 +237,7 @@ int upload_matrix(int wtype, const uint8_t* blocks, size_t rows, size_t k, DevMa
 }
 
 void free_matrix(DevMatrix* m) {
-    if (m->qs) (void)hipFree(m->qs);
-    if (m->scale) (void)hipFree(m->scale);
-    if (m->fq) (void)hipFree(m->fq);
+    if (m->qs) (void)hipFree(m->qs);  // (one allocation)
     m->qs = m->fq = nullptr;
     m->scale = m->fs = nullptr;
 }

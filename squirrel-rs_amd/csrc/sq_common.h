@@ -47,7 +47,7 @@ constexpr const char* kA32Disabled =
 // Bytes per weight are unchanged (1.0625 / 0.5625 / 2).
 //
 // Matrices that the matrix-core kernels multiply have a second copy in
-// fragment order (below): fq and fs, one allocation.
+// fragment order (below), fq and fs.  All four are one allocation, at qs.
 struct DevMatrix {
     int wtype = 0;
     int rows = 0;
@@ -55,7 +55,7 @@ struct DevMatrix {
     void* qs = nullptr;
     uint16_t* scale = nullptr;
     void* fq = nullptr;      // Q8_0: int8; Q4_0: packed nibbles of q - 8
-    uint16_t* fs = nullptr;  // (inside fq's allocation)
+    uint16_t* fs = nullptr;
     size_t payload_bytes() const;
     size_t scale_bytes() const;
 };
