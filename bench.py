@@ -52,10 +52,11 @@ ATTN_F16_PRODUCTS = 3
 # Matrix elements per layer of the 1B shape: QKV 2048x3072, o 2048x2048,
 # gate/up 2048x16384, down 8192x2048.
 MATMUL_ELEMS_PER_LAYER = 60817408
-# per output element per 32-block in the int8 matmul: the convert of the
-# integer block sum and the fused multiply-add (the scale product comes from
-# the f16 matrix instruction)
-VALU_RESCALE_OPS = 2
+# One 32x32 output tile and 32-element block of the int8 matmul (65536 ops) with
+# all its operands in registers, per SIMD: the matrix instructions, and the
+# subtraction and the fused multiply-add of each element (the scale product
+# comes from the f16 matrix instruction).  Measured.
+RESCALE_TILE_NS = 47.0
 CONFIGS = {
     "q8": dict(wtype="Q8_0", prompt=32, gen=64,
                workload="Llama-3.2-1B arch, Q8_0 GGUF, 32-token prompt then 64 greedy tokens"),
@@ -235,9 +236,9 @@ def run_workload(name: str, cfg: dict, K: int, W: int, seed: int, kernel_iters: 
         attn_flops = 4.0 * info.head_dim * S * (S + 1) / 2 * info.n_heads * L
         mm_tops = mm_ops / (ph["matmul"] / 1e3) / 1e12
         at_tflops = attn_flops / (ph["attention"] / 1e3) / 1e12
-        # VALU ceiling of the int8 matmul's per-block rescale: 256 CUs x 64
-        # lanes x 2.4 GHz element operations, VALU_RESCALE_OPS per 64 int8 ops
-        valu_ceiling = 256 * 64 * 2.4e9 / VALU_RESCALE_OPS * 64 / 1e12
+        # ceiling of the int8 matmul with its per-block rescale: 1024 SIMDs,
+        # 65536 int8 ops per RESCALE_TILE_NS each
+        valu_ceiling = 1024 * 65536 / RESCALE_TILE_NS / 1e3
         block["prefill_phases_ms"] = {k: round(v, 3) for k, v in ph.items()}
         block["prefill_mfma"] = {
             "matmul_int8_tops": round(mm_tops, 1), "matmul_frac_of_int8_peak": round(mm_tops / INT8_PEAK_TOPS, 4),
@@ -253,8 +254,8 @@ def run_workload(name: str, cfg: dict, K: int, W: int, seed: int, kernel_iters: 
             block["prefill_mfma"]["attention_frac_of_f16_mfma_peak"] = round(f16_tflops / F16_MFMA_PEAK_TFLOPS, 4)
         block["prefill_roofline"] = {"bound": "mfma", "achieved": round(mm_tops, 1), "peak": INT8_PEAK_TOPS,
                                      "unit": "TOP/s", "frac": round(mm_tops / INT8_PEAK_TOPS, 4),
-                                     "kernel": "gemm_dma_kernel (v_mfma_i32_32x32x32_i8 on 128x128 tiles staged "
-                                               "by direct global-to-LDS loads; gate/up with the fused SiLU*up "
+                                     "kernel": "gemm_tile_kernel (v_mfma_i32_32x32x32_i8 on 128x128 tiles, operands "
+                                               "loaded in fragment order; gate/up with the fused SiLU*up "
                                                "epilogue, q|k|v, o and down with K split 2-3 ways and their "
                                                "partial sums)"}
         log(f"[{name}] prefill phases {ph}; int8 matmul {mm_tops:.0f} TOP/s, attention {at_tflops:.1f} TFLOP/s")
