@@ -410,18 +410,24 @@ int ensure_prefill(sq_ctx* c, size_t n) {
     if (n <= c->cap_rows) return 0;
     const Config& g = c->m->cfg;
     const size_t D = g.dim, F = g.ffn, QD = (size_t)g.n_heads * g.head_dim, KVD = (size_t)g.n_kv_heads * g.head_dim;
-    dfree(c->p_hidden); dfree(c->p_normed); dfree(c->p_qkv); dfree(c->p_q); dfree(c->p_attn);
-    dfree(c->p_gu); dfree(c->p_act); dfree(c->p_aq); dfree(c->p_ad);
+    auto drop = [c]() {
+        c->cap_rows = 0;  // no buffers until all of the new ones are there
+        dfree(c->p_hidden); dfree(c->p_normed); dfree(c->p_qkv); dfree(c->p_q); dfree(c->p_attn);
+        dfree(c->p_gu); dfree(c->p_act); dfree(c->p_aq); dfree(c->p_ad);
+    };
+    drop();
     int st;
     const size_t wmax = std::max(std::max(D, F), QD);
     if ((st = dmalloc(&c->p_hidden, n * D)) || (st = dmalloc(&c->p_normed, n * D)) ||
         (st = dmalloc(&c->p_qkv, n * (QD + 2 * KVD))) || (st = dmalloc(&c->p_q, n * QD)) ||
         (st = dmalloc(&c->p_attn, n * QD)) || (st = dmalloc(&c->p_gu, n * 2 * F)) ||
         (st = dmalloc(&c->p_act, n * F)) || (st = dmalloc(&c->p_aq, n * wmax)) ||
-        (st = dmalloc(&c->p_ad, n * wmax / 32)))
+        (st = dmalloc(&c->p_ad, n * wmax / 32)) ||
+        (!c->p_split && (st = dmalloc(&c->p_split, kPrefillSplitFloats))) ||
+        (!c->p_kvs && (st = dmalloc(&c->p_kvs, attn_split_words((int)c->max_pos, g.n_kv_heads))))) {
+        drop();
         return st;
-    if (!c->p_split && (st = dmalloc(&c->p_split, kPrefillSplitFloats))) return st;
-    if (!c->p_kvs && (st = dmalloc(&c->p_kvs, attn_split_words((int)c->max_pos, g.n_kv_heads)))) return st;
+    }
     c->cap_rows = n;
     return 0;
 }

@@ -523,9 +523,17 @@ hipError_t hipDeviceSynchronize() {
 }
 namespace sqemu {
 uint64_t g_malloc_calls = 0;
+size_t g_dev_cap = SIZE_MAX;  // device bytes that hipMalloc may hand out together (a driver sets it)
+size_t dev_bytes() {          // live device bytes
+    size_t n = 0;
+    for (auto& b : g_dev) n += b.second;
+    return n;
+}
 }
 hipError_t hipMalloc(void** p, size_t n) {
     sqemu::g_malloc_calls++;
+    if (sqemu::g_dev_cap != SIZE_MAX && (n > sqemu::g_dev_cap || sqemu::dev_bytes() > sqemu::g_dev_cap - n))
+        return hipErrorOutOfMemory;
     // exact-size heap blocks: the sanitizer poisons everything past n
     void* q = nullptr;
     if (posix_memalign(&q, 256, n ? n : 1)) return hipErrorOutOfMemory;

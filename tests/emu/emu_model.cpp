@@ -22,6 +22,8 @@
 
 namespace sqemu {
 extern uint64_t g_malloc_calls;  // hipMalloc calls so far (tests/emu/emu.cpp)
+extern size_t g_dev_cap;         // device bytes that hipMalloc may hand out
+size_t dev_bytes();              // device bytes it has handed out
 }
 
 static void die(const char* what, int st) {
@@ -150,6 +152,40 @@ int main(int argc, char** argv) {
             sq_memcpy_h2d(d_ids, ids, sizeof(ids));
             printf("embed ids %u %u %u status %d\n", ids[0], ids[1], ids[2], sq_embed(d_ids, 3, W, d_out));
         }
+        return 0;
+    }
+    if (argc == 3 && std::string(argv[1]) == "--prefill-oom") {
+        // a prompt for whose buffers there is no room fails with a status, and
+        // so does a shorter one after it (its buffers went with the growth that
+        // failed) until there is room again
+        sq_model* m = nullptr;
+        int st = sq_model_load_gguf(argv[2], &m);
+        if (st) die("sq_model_load_gguf", st);
+        sq_model_info info;
+        sq_model_info_get(m, &info);
+        sq_ctx* c = nullptr;
+        if ((st = sq_ctx_new(m, 64, SQ_CTX_MULTI_KERNEL, &c))) die("sq_ctx_new", st);
+        std::vector<uint32_t> ids(40);
+        for (size_t i = 0; i < ids.size(); i++) ids[i] = (uint32_t)(7 * i + 3);
+        std::vector<float> want(info.vocab), got(info.vocab);
+        if ((st = sq_forward(m, c, ids.data(), 5))) die("sq_forward", st);
+        if ((st = sq_logits(c, want.data(), want.size()))) die("sq_logits", st);
+        for (int cap : {1, 1, 0}) {
+            sqemu::g_dev_cap = cap ? sqemu::dev_bytes() : SIZE_MAX;
+            if ((st = sq_ctx_reset(c))) die("sq_ctx_reset", st);
+            const int grown = sq_forward(m, c, ids.data(), ids.size());
+            if ((st = sq_ctx_reset(c))) die("sq_ctx_reset", st);
+            if (cap) sqemu::g_dev_cap = sqemu::dev_bytes();
+            const int again = sq_forward(m, c, ids.data(), 5);
+            int same = 0;
+            if (!again) {
+                if ((st = sq_logits(c, got.data(), got.size()))) die("sq_logits", st);
+                same = memcmp(got.data(), want.data(), got.size() * 4) == 0;
+            }
+            printf("room %d grown %d again %d same %d\n", !cap, grown, again, same);
+        }
+        sq_ctx_free(c);
+        sq_model_free(m);
         return 0;
     }
     if (argc < 8) {

@@ -123,6 +123,17 @@ def test_device_token_id_past_the_table_is_an_error(emu):
     assert got == [("3", "63", "0", "0"), ("3", "64", "0", "22"), ("4294967295", "1", "2", "22")], p.stdout
 
 
+def test_prefill_without_room_fails_and_recovers(emu, models):
+    """Growing a context's prefill buffers frees the old ones first.  Where
+    the new ones do not fit, that prompt and every later one, also one that
+    the old buffers held, ends with a status (64, not a launch on null
+    buffers), and with room again the prompt gives the same logits."""
+    p = subprocess.run([emu, "--prefill-oom", models["Q8_0"]], capture_output=True, text=True, env=ENV)
+    assert p.returncode == 0 and "AddressSanitizer" not in p.stderr, p.stdout + p.stderr[-2000:]
+    got = re.findall(r"^room (\d) grown (\d+) again (\d+) same (\d)$", p.stdout, re.M)
+    assert got == [("0", "64", "64", "0")] * 2 + [("1", "0", "0", "1")], p.stdout
+
+
 @pytest.mark.parametrize("case,where", [("host", "stack"), ("hoststruct", "stack"), ("freed", "heap")])
 def test_emulator_refuses_host_and_freed_pointers(emu, case, where):
     """Device memory is host memory in the emulator, so a host pointer or a
