@@ -48,12 +48,7 @@ int sq_device_count(int* n) {
 }
 
 int sq_malloc(void** p, size_t bytes) {
-    hipError_t e = hipMalloc(p, bytes ? bytes : 1);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        scratch_trim();
-        SQ_HIP_CHECK(hipMalloc(p, bytes ? bytes : 1));
-    }
+    SQ_HIP_CHECK(device_alloc(p, bytes ? bytes : 1));
     return 0;
 }
 int sq_free(void* p) {
@@ -152,7 +147,7 @@ int sq_ctx_step_trace(sq_ctx* c, int enable) {
         return 0;
     }
     const int stride = 20 * c->m->cfg.n_layers + 4;
-    if (!c->s_trace) SQ_HIP_CHECK(hipMalloc((void**)&c->s_trace, (size_t)c->step_grid * stride * 8));
+    if (!c->s_trace) SQ_HIP_CHECK(device_alloc((void**)&c->s_trace, (size_t)c->step_grid * stride * 8));
     SQ_HIP_CHECK(hipMemset(c->s_trace, 0, (size_t)c->step_grid * stride * 8));
     c->step.trace = c->s_trace;
     c->step.trace_stride = stride;

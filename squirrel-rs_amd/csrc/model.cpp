@@ -90,12 +90,7 @@ size_t gguf_row_bytes(int wtype, size_t k) {
 template <typename T>
 int dmalloc(T** p, size_t count) {
     if (count == 0) count = 1;
-    hipError_t e = hipMalloc((void**)p, count * sizeof(T));
-    if (e != hipSuccess) {  // the operators' idle scratch goes first
-        (void)hipGetLastError();
-        scratch_trim();
-        e = hipMalloc((void**)p, count * sizeof(T));
-    }
+    const hipError_t e = device_alloc((void**)p, count * sizeof(T));
     if (e != hipSuccess)
         return set_error(SQ_ERR_HIP, "hipMalloc(" + std::to_string(count * sizeof(T)) + "): " + hipGetErrorString(e));
     return 0;
@@ -908,7 +903,10 @@ int ctx_create(const sq_model* m, size_t max_pos, uint32_t flags, sq_ctx** out) 
         (st = dmalloc((uint8_t**)&c->lsm_ws, kScoreRows * (size_t)log_softmax_parts(g.vocab) * kLsmPartBytes)) || (st = dmalloc(&c->d_id_error, 2)))
         return fail(st);
     he = hipHostMalloc((void**)&c->h_pinned, (max_pos + 16) * sizeof(uint32_t), hipHostMallocDefault);
-    if (he != hipSuccess) return fail(set_error(SQ_ERR_HIP, std::string("hipHostMalloc: ") + hipGetErrorString(he)));
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(set_error(SQ_ERR_HIP, std::string("hipHostMalloc: ") + hipGetErrorString(he)));
+    }
 
     // RoPE (cos, sin) per position, computed on the host exactly as the
     // reference: theta = f32(pos) * inv_freq[j], then libm sinf / cosf
@@ -1020,10 +1018,8 @@ int ctx_score(sq_ctx* c, const uint32_t* ids, size_t n, size_t burn, double* log
                                        c->d_id_error, c->lsm_ws);
     };
     if ((st = log_probs(c->logits, 1, burn))) return st;
-    if (c->persist && !c->s_rows && dmalloc(&c->s_rows, (size_t)kScoreRows * V)) {
-        (void)hipGetLastError();  // no room: every step's row is scored in place
-        c->s_rows = nullptr;
-    }
+    if (c->persist && !c->s_rows && dmalloc(&c->s_rows, (size_t)kScoreRows * V))
+        c->s_rows = nullptr;  // no room: every step's row is scored in place
     if (c->persist && c->s_rows) {
         // Every step stays on the device, and the persistent steps run back
         // to back: step i takes its token from a second copy of the window

@@ -36,6 +36,16 @@ size_t rounded(size_t n) {
 
 }  // namespace
 
+hipError_t device_alloc(void** p, size_t n) {
+    hipError_t e = hipMalloc(p, n);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        scratch_trim();
+        if ((e = hipMalloc(p, n)) != hipSuccess) (void)hipGetLastError();
+    }
+    return e;
+}
+
 int scratch_get(size_t n, void** p, size_t* size, int* device) {
     SQ_HIP_CHECK(hipGetDevice(device));
     n = rounded(n ? n : 1);
@@ -56,12 +66,7 @@ int scratch_get(size_t n, void** p, size_t* size, int* device) {
             return 0;
         }
     }
-    hipError_t e = hipMalloc(p, n);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        scratch_trim();
-        e = hipMalloc(p, n);
-    }
+    const hipError_t e = device_alloc(p, n);
     if (e != hipSuccess) {
         *p = nullptr;
         return set_error(SQ_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));

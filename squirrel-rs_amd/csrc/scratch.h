@@ -6,6 +6,8 @@
 // stream, so a block that goes to another call, of this thread or another, is
 // written there only behind the launches that still read it.
 #pragma once
+#include <hip/hip_runtime.h>
+
 #include <cstddef>
 
 namespace sq {
@@ -17,8 +19,11 @@ constexpr unsigned kScratchAge = 256;               // an idle block is freed af
 int scratch_get(size_t n, void** p, size_t* size, int* device);
 // Back to the pool (the block's launches may still be queued on the null stream).
 void scratch_put(void* p, size_t size, int device);
-// Frees the current device's idle blocks (an allocation failed and is tried again).
+// Frees the current device's idle blocks.
 void scratch_trim();
+// hipMalloc, tried again without the idle blocks where it fails.  A failure
+// leaves no error behind for the next launch's check to find.
+hipError_t device_alloc(void** p, size_t n);
 
 // A temporary of one entry point's call.
 struct Tmp {

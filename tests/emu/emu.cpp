@@ -488,8 +488,15 @@ bool pinned(const void* p, size_t n) {
 }  // namespace
 }  // namespace sqemu
 
-hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipPeekAtLastError() { return hipSuccess; }
+// A failed call's error stays until hipGetLastError reads it, as on the device:
+// the next launch's check reports it.
+static hipError_t g_last_error = hipSuccess;
+hipError_t hipGetLastError() {
+    const hipError_t e = g_last_error;
+    g_last_error = hipSuccess;
+    return e;
+}
+hipError_t hipPeekAtLastError() { return g_last_error; }
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "emulated error"; }
 hipError_t hipGetDeviceCount(int* n) {
     *n = 1;
@@ -533,10 +540,10 @@ size_t dev_bytes() {          // live device bytes
 hipError_t hipMalloc(void** p, size_t n) {
     sqemu::g_malloc_calls++;
     if (sqemu::g_dev_cap != SIZE_MAX && (n > sqemu::g_dev_cap || sqemu::dev_bytes() > sqemu::g_dev_cap - n))
-        return hipErrorOutOfMemory;
+        return g_last_error = hipErrorOutOfMemory;
     // exact-size heap blocks: the sanitizer poisons everything past n
     void* q = nullptr;
-    if (posix_memalign(&q, 256, n ? n : 1)) return hipErrorOutOfMemory;
+    if (posix_memalign(&q, 256, n ? n : 1)) return g_last_error = hipErrorOutOfMemory;
     // device memory starts with arbitrary contents
     memset(q, 0xA5, n ? n : 1);
     *p = q;
