@@ -24,9 +24,11 @@ using namespace sq;
 
 namespace {
 
+// The end of an operator call: nothing of it is queued any more when it
+// returns, with an error (st) too.
 int finish(int st) {
+    const hipError_t e = hipStreamSynchronize(nullptr);
     if (st) return st;
-    hipError_t e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return set_error(SQ_ERR_HIP, std::string("kernel: ") + hipGetErrorString(e));
     return 0;
 }

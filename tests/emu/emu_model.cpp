@@ -133,6 +133,31 @@ int main(int argc, char** argv) {
         }
         return 0;
     }
+    if (argc == 2 && std::string(argv[1]) == "--shared-error") {
+        // sq_linear_shared whose second matrix (no rows) is refused behind the
+        // first one's launches: a call that returns leaves nothing queued
+        const int k = 96, n = 33, m = 40;
+        std::vector<uint8_t> w((size_t)n * (k / 32) * 34, 1);
+        sq_weight *W[2] = {nullptr, nullptr};
+        int st = sq_weight_upload(SQ_Q8_0, w.data(), n, k, &W[0]);
+        if (!st) st = sq_weight_upload(SQ_Q8_0, w.data(), 0, k, &W[1]);
+        if (st) die("sq_weight_upload", st);
+        float *dx = nullptr, *dy = nullptr, *dz = nullptr;
+        sq_malloc((void**)&dx, (size_t)m * k * 4);
+        sq_malloc((void**)&dy, (size_t)m * n * 4);
+        sq_malloc((void**)&dz, 4);
+        std::vector<float> x((size_t)m * k, 0.5f), y((size_t)m * n), z(y.size());
+        sq_memcpy_h2d(dx, x.data(), x.size() * 4);
+        sq_memcpy_h2d(dy, z.data(), z.size() * 4);
+        sq_synchronize();
+        float* const outs[2] = {dy, dz};
+        st = sq_linear_shared(dx, m, k, W, outs, 2, 0);
+        memcpy(y.data(), dy, y.size() * 4);  // (no runtime call that would wait)
+        sq_synchronize();
+        sq_memcpy_d2h(z.data(), dy, z.size() * 4);
+        printf("shared status %d left_queued %d\n", st, memcmp(y.data(), z.data(), y.size() * 4) != 0);
+        return 0;
+    }
     if (argc == 2 && std::string(argv[1]) == "--embed-guard") {
         // sq_embed with device ids in and past a 64-row Q8_0 table: the
         // in-range call succeeds; an id of 64 or of 2^32 - 1 is SQ_ERR_ARG

@@ -123,6 +123,15 @@ def test_device_token_id_past_the_table_is_an_error(emu):
     assert got == [("3", "63", "0", "0"), ("3", "64", "0", "22"), ("4294967295", "1", "2", "22")], p.stdout
 
 
+def test_failed_shared_linear_leaves_nothing_queued(emu):
+    """linear_shared whose second matrix is refused: when the status comes
+    back, the first product's launches are no longer writing its output."""
+    p = subprocess.run([emu, "--shared-error"], capture_output=True, text=True, env=ENV)
+    assert p.returncode == 0 and "AddressSanitizer" not in p.stderr, p.stdout + p.stderr[-2000:]
+    m = re.search(r"^shared status (\d+) left_queued (\d)$", p.stdout, re.M)
+    assert m and int(m[1]) != 0 and m[2] == "0", p.stdout
+
+
 def test_prefill_without_room_fails_and_recovers(emu, models):
     """Growing a context's prefill buffers frees the old ones first.  Where
     the new ones do not fit, that prompt and every later one, also one that
