@@ -924,7 +924,7 @@ int run_rows_shared(hipStream_t s, const DevMatrix* const* ws, int n, const int8
         gx += (ws[i]->rows + 31) / 32;
         count_launch(1, 32);
     }
-    for (int i = n - 1; i < kSharedMax - 1; i++) more.begin[i] = INT32_MAX;
+    for (int i = n - 1; i < kSharedMax - 1; i++) more.begin[i] = gx;  // (past the grid)
     const int KB = ws[0]->k / 32;
     hipLaunchKernelGGL((gemm_rows_kernel<WT, 1, RW_NB, RW_SHARED>), dim3(gx, (m + 31) / 32), dim3(RW_NW * 64), 0, s,
                        frag(*ws[0]), aq, ad, m, outs[0], ws[0]->rows, 0, rows_per_wave(KB, RW_NB), KB, (size_t)0,
@@ -1131,6 +1131,11 @@ int launch_gemm_shared(hipStream_t s, const DevMatrix* const* ws, int n, const i
             return -1;
         const RowsPlan p = rows_plan(w, m, true, kGemmSplitFloats);
         if (p.two || p.splits != 1) return -1;
+        // outputs that share memory are written in their order, launch by launch
+        for (int j = 0; j < i; j++)
+            if ((uintptr_t)outs[i] < (uintptr_t)(outs[j] + (size_t)m * ws[j]->rows) &&
+                (uintptr_t)outs[j] < (uintptr_t)(outs[i] + (size_t)m * w.rows))
+                return -1;
     }
     if (ws[0]->wtype == WT_Q8_0) return run_rows_shared<WT_Q8_0>(s, ws, n, aq, ad, m, outs);
     if (ws[0]->wtype == WT_Q4_0) return run_rows_shared<WT_Q4_0>(s, ws, n, aq, ad, m, outs);

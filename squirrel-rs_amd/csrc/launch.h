@@ -187,7 +187,8 @@ int launch_gemm(hipStream_t s, const DevMatrix& w, bool a8, const int8_t* aq, co
                 const float* x, int m, float* out, int ldo, bool accumulate,
                 float* ws = nullptr, size_t ws_floats = 0, const NormThen* then = nullptr);
 // The products of one input with n matrices of equal k in one launch, where
-// the few-rows kernel takes each of them unsplit with a tile per workgroup:
+// the few-rows kernel takes each of them unsplit with a tile per workgroup and
+// no two outputs share memory:
 // what launch_gemm writes for each with the same workspace size, bit for bit.
 // Returns -1 (nothing launched) where that does not apply.
 constexpr int kSharedMax = 4;

@@ -255,10 +255,13 @@ void run_grid(dim3 grid, dim3 block, size_t dyn_bytes, const std::function<void(
     g_blockdim = block;
     g_dyn_bytes = dyn_bytes;
     g_dyn.assign(dyn_bytes ? dyn_bytes : 1, 0);
+    // SQEMU_REVERSE=1: the last workgroup first (their order is not defined)
+    const char* rev = getenv("SQEMU_REVERSE");
+    const bool reverse = rev && !strcmp(rev, "1");
     for (unsigned bz = 0; bz < grid.z; bz++)
         for (unsigned by = 0; by < grid.y; by++)
             for (unsigned bx = 0; bx < grid.x; bx++) {
-                g_block = dim3(bx, by, bz);
+                g_block = reverse ? dim3(grid.x - 1 - bx, grid.y - 1 - by, grid.z - 1 - bz) : dim3(bx, by, bz);
                 g_fibers.assign(nt, FiberRec{});
                 g_waves.assign(nwaves, Wave{});
                 g_blk = Block{};

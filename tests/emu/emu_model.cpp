@@ -158,6 +158,34 @@ int main(int argc, char** argv) {
         printf("shared status %d left_queued %d\n", st, memcmp(y.data(), z.data(), y.size() * 4) != 0);
         return 0;
     }
+    if (argc == 2 && std::string(argv[1]) == "--shared-overlap") {
+        // sq_linear_shared with outputs that share memory: the second product
+        // of m x n starts at row 1 of the first
+        const int k = 128, n = 40, m = 3;
+        std::vector<uint8_t> w[2];
+        sq_weight *W[2] = {nullptr, nullptr};
+        int st = 0;
+        for (int i = 0; i < 2; i++) {
+            w[i].assign((size_t)n * (k / 32) * 34, (uint8_t)(3 + 5 * i));
+            for (size_t b = 0; b < w[i].size(); b += 34) memset(&w[i][b], 0x30, 2);
+            if ((st = sq_weight_upload(SQ_Q8_0, w[i].data(), n, k, &W[i]))) die("sq_weight_upload", st);
+        }
+        float *dx = nullptr, *dy = nullptr, *dz = nullptr;
+        sq_malloc((void**)&dx, (size_t)m * k * 4);
+        sq_malloc((void**)&dy, (size_t)(m + 1) * n * 4);
+        sq_malloc((void**)&dz, (size_t)(m + 1) * n * 4);
+        std::vector<float> x((size_t)m * k), y((size_t)(m + 1) * n), z(y.size());
+        for (size_t i = 0; i < x.size(); i++) x[i] = (float)((int)(i % 13) - 5);
+        sq_memcpy_h2d(dx, x.data(), x.size() * 4);
+        for (int i = 0; i < 2; i++)
+            if ((st = sq_linear(dx, m, k, W[i], dz + i * n, 0))) die("sq_linear", st);
+        float* const outs[2] = {dy, dy + n};
+        if ((st = sq_linear_shared(dx, m, k, W, outs, 2, 0))) die("sq_linear_shared", st);
+        sq_memcpy_d2h(y.data(), dy, y.size() * 4);
+        sq_memcpy_d2h(z.data(), dz, z.size() * 4);
+        printf("overlap same %d\n", memcmp(y.data(), z.data(), y.size() * 4) == 0);
+        return 0;
+    }
     if (argc == 2 && std::string(argv[1]) == "--embed-guard") {
         // sq_embed with device ids in and past a 64-row Q8_0 table: the
         // in-range call succeeds; an id of 64 or of 2^32 - 1 is SQ_ERR_ARG

@@ -132,6 +132,15 @@ def test_failed_shared_linear_leaves_nothing_queued(emu):
     assert m and int(m[1]) != 0 and m[2] == "0", p.stdout
 
 
+@pytest.mark.parametrize("reverse", ["0", "1"])
+def test_shared_linear_with_overlapping_outputs(emu, reverse):
+    """Outputs of linear_shared that share memory hold what separate calls in
+    the same order leave there, whatever order a launch's workgroups run in."""
+    p = subprocess.run([emu, "--shared-overlap"], capture_output=True, text=True, env={**ENV, "SQEMU_REVERSE": reverse})
+    assert p.returncode == 0 and "AddressSanitizer" not in p.stderr, p.stdout + p.stderr[-2000:]
+    assert "overlap same 1" in p.stdout, p.stdout
+
+
 def test_prefill_without_room_fails_and_recovers(emu, models):
     """Growing a context's prefill buffers frees the old ones first.  Where
     the new ones do not fit, that prompt and every later one, also one that
