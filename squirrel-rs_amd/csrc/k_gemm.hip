@@ -1017,6 +1017,29 @@ int run_integer(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint1
     return run_tiles<WT>(s, t.shape, w, aq, ad, m, out, ldo, acc, t.splits, ws, then);
 }
 
+// A matrix without a fragment-order copy (there was no room for it): the copy
+// of as many rows as the workspace holds at a time, each slab's product unsplit.
+template <int WT>
+int run_slabs(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint16_t* ad, int m, float* out, int ldo,
+              bool acc, float* ws, size_t ws_floats) {
+    const size_t KB = w.k / 32, pay = KB * (WT == WT_Q8_0 ? 32 : 16), room = ws ? ws_floats * sizeof(float) : 0;
+    size_t slab = room > 256 ? (room - 256) / (pay + 2 * KB) : 0;  // (256: the scales' boundary)
+    if (slab >= 32) slab &= ~(size_t)31;
+    if (slab == 0) return set_error(SQ_ERR_HIP, "gemm: the matrix has no fragment-order copy and the workspace no room for a row");
+    for (size_t n0 = 0; n0 < (size_t)w.rows; n0 += slab) {
+        DevMatrix part = w;
+        part.rows = (int)min(slab, (size_t)w.rows - n0);
+        part.qs = (uint8_t*)w.qs + n0 * pay;
+        part.scale = w.scale + n0 * KB;
+        part.fq = ws;
+        part.fs = (uint16_t*)((uint8_t*)ws + (part.rows * pay + 255) / 256 * 256);
+        if (const int st = launch_frag_copy(s, part)) return st;
+        const NormThen* none = nullptr;
+        if (const int st = run_integer<WT>(s, part, aq, ad, m, out + n0, ldo, acc, nullptr, 0, &none)) return st;
+    }
+    return 0;
+}
+
 // SQUIRREL_PREFILL_UNFUSED=1 turns the fused gate/up and q|k|v epilogues
 // off (a test aid: the separate kernels give the same bits).
 bool prefill_fusion_enabled() {
@@ -1172,10 +1195,12 @@ int launch_gemm(hipStream_t s, const DevMatrix& w, bool a8, const int8_t* aq, co
                 int m, float* out, int ldo, bool accumulate, float* ws, size_t ws_floats, const NormThen* then) {
     if (w.k <= 0 || w.k % 32 != 0) return set_error(SQ_ERR_SHAPE, "gemm: k must be a positive multiple of 32");
     if (m <= 0) return set_error(SQ_ERR_EMPTY, "gemm: no rows");
-    if (a8 && w.wtype != WT_BF16 && w.fq == nullptr)
-        return set_error(SQ_ERR_ARG, "gemm: the matrix has no fragment-order copy");
+    if (w.rows <= 0) return set_error(SQ_ERR_SHAPE, "gemm: the matrix has no rows");
     if (a8 && (w.wtype == WT_Q8_0 || w.wtype == WT_Q4_0)) {
-        const int st = w.wtype == WT_Q8_0
+        const int st = w.fq == nullptr
+                           ? (w.wtype == WT_Q8_0 ? run_slabs<WT_Q8_0>(s, w, aq, ad, m, out, ldo, accumulate, ws, ws_floats)
+                                                 : run_slabs<WT_Q4_0>(s, w, aq, ad, m, out, ldo, accumulate, ws, ws_floats))
+                       : w.wtype == WT_Q8_0
                            ? run_integer<WT_Q8_0>(s, w, aq, ad, m, out, ldo, accumulate, ws, ws_floats, &then)
                            : run_integer<WT_Q4_0>(s, w, aq, ad, m, out, ldo, accumulate, ws, ws_floats, &then);
         if (st || !then) return st;

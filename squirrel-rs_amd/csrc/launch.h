@@ -175,7 +175,8 @@ int launch_log_softmax_rows(hipStream_t s, const float* logits, size_t stride, i
 // norm of the output rows that follows, in the launch that sums a K split where
 // there is one.
 // ws: room for ws_floats floats of partial tiles, for a K split of the
-// integer path when the output has few tiles (null: no split).
+// integer path when the output has few tiles (null: no split), or for the
+// fragment order of some of a matrix's rows where it has no copy (w.fq null).
 constexpr size_t kGemmSplitFloats = (size_t)4 << 20;
 // The model context's K-split workspace: three partial 2048 x 2048 tiles
 // (the FFN down projection of a 2048-token prompt) and more.

@@ -213,8 +213,12 @@ int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts, const st
         }
         r0 += rows[p];
     }
-    int st;
-    if ((st = dmalloc((uint8_t**)&out->qs, frag ? f_off + up256(q_bytes) + s_bytes : h.size()))) return st;
+    int st = dmalloc((uint8_t**)&out->qs, frag ? f_off + up256(q_bytes) + s_bytes : h.size());
+    if (st && frag) {  // room for one copy only: the matmul makes the other as it goes (launch_gemm)
+        frag = false;
+        st = dmalloc((uint8_t**)&out->qs, h.size());
+    }
+    if (st) return st;
     if (!h.empty()) SQ_HIP_CHECK(hipMemcpy(out->qs, h.data(), h.size(), hipMemcpyHostToDevice));
     if (s_bytes) out->scale = (uint16_t*)((uint8_t*)out->qs + s_off);
     if (frag) {
@@ -260,7 +264,7 @@ int get_tensor(const GGUFFile& f, const std::string& name, const std::vector<uin
 
 }  // namespace
 
-int model_load_impl(const char* path, sq_model** out, bool upload) {
+int model_load_impl(const char* path, sq_model** out, bool upload, bool frag) {
     GGUFFile f;
     int st = f.open(path);
     if (st) return st;
@@ -354,10 +358,10 @@ int model_load_impl(const char* path, sq_model** out, bool upload) {
         Layer& L = m->layers[i];
         const LayerSrc& S = src[i];
         if ((st = up_norm(S.an, &L.attn_norm)) || (st = up_norm(S.fn, &L.ffn_norm)) ||
-            (st = upload_stacked(wtype, {S.wq, S.wk, S.wv}, {QD, KVD, KVD}, D, &L.qkv, true)) ||
-            (st = upload_matrix(wtype, S.wo, D, QD, &L.o, true)) ||
-            (st = upload_stacked(wtype, {S.wg, S.wu}, {F, F}, D, &L.gateup, true)) ||
-            (st = upload_matrix(wtype, S.wd, D, F, &L.down, true)))
+            (st = upload_stacked(wtype, {S.wq, S.wk, S.wv}, {QD, KVD, KVD}, D, &L.qkv, frag)) ||
+            (st = upload_matrix(wtype, S.wo, D, QD, &L.o, frag)) ||
+            (st = upload_stacked(wtype, {S.wg, S.wu}, {F, F}, D, &L.gateup, frag)) ||
+            (st = upload_matrix(wtype, S.wd, D, F, &L.down, frag)))
             return fail(st);
         m->weight_bytes += L.qkv.payload_bytes() + L.qkv.scale_bytes() + L.o.payload_bytes() +
                            L.o.scale_bytes() + L.gateup.payload_bytes() + L.gateup.scale_bytes() +
@@ -376,8 +380,12 @@ int model_load_impl(const char* path, sq_model** out, bool upload) {
     return 0;
 }
 
-int model_load(const char* path, sq_model** out) { return model_load_impl(path, out, true); }
-int model_inspect(const char* path, sq_model** out) { return model_load_impl(path, out, false); }
+int model_load(const char* path, sq_model** out) {
+    const int st = model_load_impl(path, out, true, true);
+    // (the first matrices' second copies may have taken the last ones' room)
+    return st == SQ_ERR_HIP ? model_load_impl(path, out, true, false) : st;
+}
+int model_inspect(const char* path, sq_model** out) { return model_load_impl(path, out, false, false); }
 
 void model_free(sq_model* m) {
     if (!m) return;

@@ -27,7 +27,7 @@ void rope_inv_freq(int head_dim, float base, float factor, float low, float high
                    float* out);
 
 // Upload `rows` rows of GGUF blocks into the device layout (DevMatrix), with
-// frag also in fragment order (quantized types).
+// frag also in fragment order (quantized types, where there is room for both).
 int upload_matrix(int wtype, const uint8_t* blocks, size_t rows, size_t k, DevMatrix* out, bool frag);
 // Upload several GGUF matrices with equal k as one stacked device matrix.
 int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts,

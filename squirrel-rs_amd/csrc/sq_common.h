@@ -47,7 +47,8 @@ constexpr const char* kA32Disabled =
 // Bytes per weight are unchanged (1.0625 / 0.5625 / 2).
 //
 // Matrices that the matrix-core kernels multiply have a second copy in
-// fragment order (below), fq and fs.  All four are one allocation, at qs.
+// fragment order (below), fq and fs (null where the device had no room for
+// it).  All four are one allocation, at qs.
 struct DevMatrix {
     int wtype = 0;
     int rows = 0;

@@ -207,6 +207,80 @@ int main(int argc, char** argv) {
         }
         return 0;
     }
+    if (argc == 4 && std::string(argv[1]) == "--no-copy-linear") {
+        // sq_linear and sq_linear_noalloc with a weight whose fragment-order
+        // copy does not fit, against the same weight with its copy
+        const int wt = atoi(argv[2]), k = atoi(argv[3]), n = 100;
+        const size_t bb = wt == SQ_Q8_0 ? 34 : 18;
+        std::mt19937 rng(3);
+        std::vector<uint8_t> w((size_t)n * (k / 32) * bb);
+        for (size_t i = 0; i < w.size(); i++) w[i] = (uint8_t)rng();
+        for (size_t b = 0; b < w.size(); b += bb) {
+            const uint16_t d = or_f32_to_f16(0.001f + 0.002f * (float)(rng() % 1000) / 1000.0f);
+            memcpy(&w[b], &d, 2);
+        }
+        sq_weight *W = nullptr, *V = nullptr;
+        int st = sq_weight_upload(wt, w.data(), n, k, &W);
+        if (st) die("sq_weight_upload", st);
+        float *dx = nullptr, *dy = nullptr;
+        sq_malloc((void**)&dx, (size_t)70 * k * 4);
+        sq_malloc((void**)&dy, (size_t)70 * n * 4);
+        std::vector<float> x((size_t)70 * k), y((size_t)70 * n), z(y.size());
+        std::normal_distribution<float> nd(0.0f, 1.0f);
+        for (auto& v : x) v = nd(rng);
+        sq_memcpy_h2d(dx, x.data(), x.size() * 4);
+        sqemu::g_dev_cap = sqemu::dev_bytes() + w.size() + 512;  // (512: the parts' 256-byte boundaries)
+        st = sq_weight_upload(wt, w.data(), n, k, &V);
+        sqemu::g_dev_cap = SIZE_MAX;
+        if (st) die("sq_weight_upload without room for the copy", st);
+        for (int m : k < 4096 ? std::vector<int>{1, 5, 70} : std::vector<int>{5})  // (long rows take long here)
+            for (int noalloc = 0; noalloc < (k < 4096 ? 2 : 1); noalloc++) {
+                auto* const f = noalloc ? sq_linear_noalloc : sq_linear;
+                if ((st = f(dx, m, k, W, dy, 0))) die("linear", st);
+                sq_memcpy_d2h(y.data(), dy, (size_t)m * n * 4);
+                sq_memset(dy, 0xFF, (size_t)m * n * 4);
+                if ((st = f(dx, m, k, V, dy, 0))) die("linear without the copy", st);
+                sq_memcpy_d2h(z.data(), dy, (size_t)m * n * 4);
+                double num = 0, den = 0;
+                for (size_t i = 0; i < (size_t)m * n; i++) {
+                    num += ((double)y[i] - z[i]) * ((double)y[i] - z[i]);
+                    den += (double)y[i] * y[i];
+                }
+                printf("nocopy m %d noalloc %d rel %.3e\n", m, noalloc, std::sqrt(num / den));
+            }
+        return 0;
+    }
+    if (argc == 3 && std::string(argv[1]) == "--no-copy-model") {
+        // a model for whose fragment-order copies there is no room loads and
+        // prefills without them
+        std::vector<float> logits[2];
+        for (int i = 0; i < 2; i++) {
+            sq_model* m = nullptr;
+            int st = sq_model_load_gguf(argv[2], &m);
+            if (st) die("sq_model_load_gguf", st);
+            const size_t held = sqemu::dev_bytes();
+            sqemu::g_dev_cap = SIZE_MAX;
+            sq_model_info info;
+            sq_model_info_get(m, &info);
+            sq_ctx* c = nullptr;
+            if ((st = sq_ctx_new(m, 64, SQ_CTX_MULTI_KERNEL, &c))) die("sq_ctx_new", st);
+            std::vector<uint32_t> ids(40);
+            for (size_t k = 0; k < ids.size(); k++) ids[k] = (uint32_t)(7 * k + 3);
+            logits[i].resize(info.vocab);
+            if ((st = sq_forward(m, c, ids.data(), ids.size()))) die("sq_forward", st);
+            if ((st = sq_logits(c, logits[i].data(), info.vocab))) die("sq_logits", st);
+            sq_ctx_free(c);
+            sq_model_free(m);
+            sqemu::g_dev_cap = held - 1;  // one byte less than with the copies
+        }
+        double num = 0, den = 0;
+        for (size_t k = 0; k < logits[0].size(); k++) {
+            num += ((double)logits[0][k] - logits[1][k]) * ((double)logits[0][k] - logits[1][k]);
+            den += (double)logits[0][k] * logits[0][k];
+        }
+        printf("nocopy model rel %.3e\n", std::sqrt(num / den));
+        return 0;
+    }
     if (argc == 3 && std::string(argv[1]) == "--prefill-oom") {
         // a prompt for whose buffers there is no room fails with a status, and
         // so does a shorter one after it (its buffers went with the growth that

@@ -123,6 +123,30 @@ def test_device_token_id_past_the_table_is_an_error(emu):
     assert got == [("3", "63", "0", "0"), ("3", "64", "0", "22"), ("4294967295", "1", "2", "22")], p.stdout
 
 
+@pytest.mark.parametrize("wtype,k", [(Q8_0, 96), (Q4_0, 96), (Q4_0, 2048), (Q8_0, 160 * 1024)])
+def test_weight_without_room_for_its_copy(emu, wtype, k):
+    """A weight that fits the device once and not twice uploads and multiplies
+    as one with its fragment-order copy does, within the reordering of a K
+    split's f32 sums (4e-6 of the terms, as between the tilings); K = 160 Ki
+    takes two slabs of rows through the workspace."""
+    p = subprocess.run([emu, "--no-copy-linear", str(wtype), str(k)], capture_output=True, text=True, env=ENV)
+    assert "AddressSanitizer" not in p.stderr, p.stderr[-2000:]
+    assert p.returncode == 0, p.stdout + p.stderr[-2000:]
+    got = re.findall(r"^nocopy m (\d+) noalloc (\d) rel (\S+)$", p.stdout, re.M)
+    assert len(got) == (6 if k < 4096 else 1) and all(float(r) < 4e-6 for _, _, r in got), p.stdout
+
+
+def test_model_without_room_for_copies(emu, models):
+    """A model that fits only without its fragment-order copies loads, and its
+    prompt gives the logits of the model with them, to the quantization steps
+    that reordered sums move (up to 1.7e-2 of the logits between two orders on
+    the 1B shape)."""
+    p = subprocess.run([emu, "--no-copy-model", models["Q8_0"]], capture_output=True, text=True, env=ENV)
+    assert p.returncode == 0 and "AddressSanitizer" not in p.stderr, p.stdout + p.stderr[-2000:]
+    m = re.search(r"^nocopy model rel (\S+)$", p.stdout, re.M)
+    assert m and float(m[1]) < 3e-2, p.stdout
+
+
 def test_failed_shared_linear_leaves_nothing_queued(emu):
     """linear_shared whose second matrix is refused: when the status comes
     back, the first product's launches are no longer writing its output."""
