@@ -69,6 +69,9 @@ int sq_memcpy_h2d(void* d_dst, const void* src, size_t bytes);
 int sq_memcpy_d2h(void* dst, const void* d_src, size_t bytes);
 int sq_memset(void* d_dst, int value, size_t bytes);
 int sq_synchronize(void);
+/* No counterpart in the reference: the operator-level calls keep up to 256 MB
+ * of idle scratch per device between calls; this frees the current device's. */
+int sq_scratch_trim(void);
 
 /* ---- GGUF files --------------------------------------------------------
  * Synthetic Llama GGUF writer: the seeded random-init models the benchmarks

@@ -74,6 +74,11 @@ int sq_synchronize(void) {
     return 0;
 }
 
+int sq_scratch_trim(void) {
+    scratch_trim();
+    return 0;
+}
+
 int sq_synth_write_gguf(const char* path, const sq_synth_spec* spec) {
     if (!path || !spec) return set_error(SQ_ERR_ARG, "synth: null argument");
     return synth_write(path, *spec);

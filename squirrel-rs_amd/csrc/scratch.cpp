@@ -48,7 +48,8 @@ hipError_t device_alloc(void** p, size_t n) {
 
 int scratch_get(size_t n, void** p, size_t* size, int* device) {
     SQ_HIP_CHECK(hipGetDevice(device));
-    n = rounded(n ? n : 1);
+    const size_t want = n ? n : 1;
+    n = want > kScratchKeep ? want : rounded(want);  // (larger blocks are never kept)
     if (*device >= 0 && *device < kMaxDevices) {
         Pool& P = pool_of(*device);
         std::lock_guard<std::mutex> lk(P.mu);
@@ -66,7 +67,11 @@ int scratch_get(size_t n, void** p, size_t* size, int* device) {
             return 0;
         }
     }
-    const hipError_t e = device_alloc(p, n);
+    hipError_t e = device_alloc(p, n);
+    if (e != hipSuccess && n > want) {  // rounding must not refuse what fits
+        n = want;
+        e = device_alloc(p, n);
+    }
     if (e != hipSuccess) {
         *p = nullptr;
         return set_error(SQ_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));

@@ -46,6 +46,7 @@ PROTOS = {
     "sq_memcpy_d2h": ([vp, vp, sz], i32),
     "sq_memset": ([vp, i32, sz], i32),
     "sq_synchronize": ([], i32),
+    "sq_scratch_trim": ([], i32),
     "sq_synth_write_gguf": ([C.c_char_p, C.POINTER(SynthSpec)], i32),
     "sq_gguf_inspect": ([C.c_char_p, C.POINTER(ModelInfo), vp, sz], i32),
     "sq_model_load_gguf": ([C.c_char_p, C.POINTER(vp)], i32),

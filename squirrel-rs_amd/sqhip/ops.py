@@ -181,6 +181,12 @@ def gemm_counters(reset: bool = False) -> dict:
             "max_splits": int(out[3]), "tile128x64_launches": int(out[4]), "rows_launches": int(out[5])}
 
 
+def scratch_trim() -> None:
+    """Frees the operator calls' idle scratch on the current device (up to
+    256 MB), for an allocator of the process that needs the room."""
+    check(lib().sq_scratch_trim())
+
+
 def log_softmax_at(logits: DeviceArray, idx: int) -> float:
     """log p(idx) under softmax(logits) in f64 (perplexity.rs:112-117)."""
     v = C.c_double()

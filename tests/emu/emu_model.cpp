@@ -19,6 +19,7 @@
 #include "../../include/squirrel_hip.h"
 #include "../../oracle/oracle.h"
 #include "gguf.h"
+#include "scratch.h"
 
 namespace sqemu {
 extern uint64_t g_malloc_calls;  // hipMalloc calls so far (tests/emu/emu.cpp)
@@ -205,6 +206,45 @@ int main(int argc, char** argv) {
             sq_memcpy_h2d(d_ids, ids, sizeof(ids));
             printf("embed ids %u %u %u status %d\n", ids[0], ids[1], ids[2], sq_embed(d_ids, 3, W, d_out));
         }
+        return 0;
+    }
+    if (argc == 2 && std::string(argv[1]) == "--scratch") {
+        // the pool of operator scratch: what it keeps and what it gives back
+        const size_t MB = (size_t)1 << 20, base = sqemu::dev_bytes();
+        auto get = [](size_t n) {
+            auto* t = new sq::Tmp();
+            if (int st = t->alloc(n)) die("scratch", st);
+            return t;
+        };
+        auto held = [base]() { return sqemu::dev_bytes() - base; };
+        sq::Tmp* a = get(4 * MB);
+        void* const p = a->p;
+        delete a;
+        a = get(4 * MB - 9);
+        printf("scratch reused %d\n", a->p == p && held() == 4 * MB);
+        delete a;
+        a = get(MB);  // (a block of more than twice the size is not taken)
+        printf("scratch fits %d\n", a->p != p);
+        delete a;
+        for (unsigned i = 0; i < sq::kScratchAge; i++) delete get(8192);
+        printf("scratch aged %zu\n", held());
+        std::vector<sq::Tmp*> many;
+        for (int i = 0; i < 6; i++) many.push_back(get(64 * MB));
+        for (sq::Tmp* t : many) delete t;
+        printf("scratch kept %d\n", held() <= sq::kScratchKeep && held() > sq::kScratchKeep - 64 * MB);
+        delete get(sq::kScratchKeep + 1);
+        printf("scratch large %d\n", held() <= sq::kScratchKeep);
+        sqemu::g_dev_cap = sqemu::dev_bytes();
+        void* q = nullptr;
+        const int st = sq_malloc(&q, 100 * MB);  // only where the idle blocks are
+        printf("scratch given %d\n", st);
+        sq_free(q);
+        sqemu::g_dev_cap = base + 97 * MB;  // the pool's sizes step by 8 MB here
+        a = get(97 * MB);
+        printf("scratch exact %zu\n", held() / MB);
+        delete a;
+        sqemu::g_dev_cap = SIZE_MAX;
+        printf("scratch trim %d %zu\n", sq_scratch_trim(), held());
         return 0;
     }
     if (argc == 4 && std::string(argv[1]) == "--no-copy-linear") {

@@ -123,6 +123,18 @@ def test_device_token_id_past_the_table_is_an_error(emu):
     assert got == [("3", "63", "0", "0"), ("3", "64", "0", "22"), ("4294967295", "1", "2", "22")], p.stdout
 
 
+def test_scratch_pool_bounds(emu):
+    """The operators' scratch: blocks are reused for sizes down to half
+    theirs, an idle block is freed after kScratchAge returns, at most
+    kScratchKeep bytes stay idle and larger blocks are never kept, an
+    allocation that fails takes the idle blocks, one that only fits unrounded
+    is made unrounded, and sq_scratch_trim frees what is idle."""
+    p = subprocess.run([emu, "--scratch"], capture_output=True, text=True, env=ENV)
+    assert p.returncode == 0 and "AddressSanitizer" not in p.stderr, p.stdout + p.stderr[-2000:]
+    assert re.findall(r"^scratch (.*)$", p.stdout, re.M) == [
+        "reused 1", "fits 1", "aged 8192", "kept 1", "large 1", "given 0", "exact 97", "trim 0 0"], p.stdout
+
+
 @pytest.mark.parametrize("wtype,k", [(Q8_0, 96), (Q4_0, 96), (Q4_0, 2048), (Q8_0, 160 * 1024)])
 def test_weight_without_room_for_its_copy(emu, wtype, k):
     """A weight that fits the device once and not twice uploads and multiplies
