@@ -839,6 +839,9 @@ int setup_persistent(sq_ctx* c) {
     a.stream_stride = decode_stream_stride(m->wtype, g.n_layers, g.dim, g.ffn, g.n_heads, g.n_kv_heads, g.vocab, grid);
     if ((st = dmalloc(&c->s_stream, a.stream_stride * 16 * (size_t)grid))) return st;
     a.stream = c->s_stream;
+    // the table and the matrices came over the null stream, which does not
+    // order this context's own
+    SQ_HIP_CHECK(hipDeviceSynchronize());
     if ((st = launch_build_stream(c->stream, m->wtype, a, grid, c->s_stream))) return st;
     SQ_HIP_CHECK(hipStreamSynchronize(c->stream));
     c->step_grid = grid;

@@ -208,6 +208,18 @@ int main(int argc, char** argv) {
         }
         return 0;
     }
+    if (argc == 3 && std::string(argv[1]) == "--step-setup") {
+        // a context with the persistent step is set up (SQEMU_STEP=1)
+        sq_model* m = nullptr;
+        int st = sq_model_load_gguf(argv[2], &m);
+        if (st) die("sq_model_load_gguf", st);
+        sq_ctx* c = nullptr;
+        if ((st = sq_ctx_new(m, 64, 0, &c))) die("sq_ctx_new", st);
+        printf("step set up %d\n", sq_ctx_decode_kernel(c));
+        sq_ctx_free(c);
+        sq_model_free(m);
+        return 0;
+    }
     if (argc == 2 && std::string(argv[1]) == "--scratch") {
         // the pool of operator scratch: what it keeps and what it gives back
         const size_t MB = (size_t)1 << 20, base = sqemu::dev_bytes();

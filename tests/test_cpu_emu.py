@@ -123,6 +123,15 @@ def test_device_token_id_past_the_table_is_an_error(emu):
     assert got == [("3", "63", "0", "0"), ("3", "64", "0", "22"), ("4294967295", "1", "2", "22")], p.stdout
 
 
+def test_step_setup_waits_for_its_tables(emu, models):
+    """The weight-stream builder runs on the context's own stream, which the
+    null stream's copies do not order: the layer table it reads has to have
+    arrived."""
+    p = subprocess.run([emu, "--step-setup", models["Q8_0"]], capture_output=True, text=True,
+                       env={**ENV, "SQEMU_STEP": "1"})
+    assert p.returncode == 0 and "step set up 1" in p.stdout, p.stdout + p.stderr[-2000:]
+
+
 def test_scratch_pool_bounds(emu):
     """The operators' scratch: blocks are reused for sizes down to half
     theirs, an idle block is freed after kScratchAge returns, at most
