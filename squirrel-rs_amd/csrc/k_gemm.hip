@@ -831,7 +831,8 @@ int launch_shape(hipStream_t s, int shape, const DevMatrix& w, const int8_t* aq,
 }
 
 // Blocks per split and the splits that leaves, for `splits` splits of K in
-// whole groups of four blocks.
+// whole groups of four blocks (the loop's; three splits of 64 blocks are 24, 24
+// and 16).  The parts fix the order of the sums and so a product's last bits.
 void k_partition(int KB, int* splits, int* kbs) {
     const int groups = (KB + 3) / 4;
     *kbs = ((groups + *splits - 1) / *splits) * 4;

@@ -208,6 +208,52 @@ int main(int argc, char** argv) {
         }
         return 0;
     }
+    if (argc == 7 && std::string(argv[1]) == "--split-bits") {
+        // sq_linear (Q8_0) against its sums formed here in a stated order, bit
+        // for bit: K in parts of <kbs> blocks (the last one shorter), each
+        // part's blocks folded in order by fma(f32(isum), sa * sw, acc), the
+        // parts added in order: --split-bits <m> <k> <n> <kbs> <seed>
+        const int m = atoi(argv[2]), k = atoi(argv[3]), n = atoi(argv[4]), kbs = atoi(argv[5]), KB = k / 32;
+        std::mt19937 rng((unsigned)atoi(argv[6]));
+        std::normal_distribution<float> nd(0.0f, 1.0f);
+        std::vector<float> wf((size_t)n * k), x((size_t)m * k), got((size_t)m * n);
+        for (auto& v : wf) v = nd(rng) * 0.02f;
+        for (auto& v : x) v = nd(rng);
+        std::vector<or_block_q8_0> w((size_t)n * KB), a((size_t)m * KB);
+        or_quantize_row_q8_0(wf.data(), wf.size(), w.data());
+        or_quantize_row_q8_0(x.data(), x.size(), a.data());
+        sq_weight* W = nullptr;
+        int st = sq_weight_upload(SQ_Q8_0, w.data(), n, k, &W);
+        if (st) die("sq_weight_upload", st);
+        float *dx = nullptr, *dy = nullptr;
+        sq_malloc((void**)&dx, x.size() * 4);
+        sq_malloc((void**)&dy, got.size() * 4);
+        sq_memcpy_h2d(dx, x.data(), x.size() * 4);
+        sq_gemm_counters(1, nullptr);
+        if ((st = sq_linear(dx, m, k, W, dy, 0))) die("sq_linear", st);
+        uint64_t gc[6];
+        sq_gemm_counters(0, gc);
+        sq_memcpy_d2h(got.data(), dy, got.size() * 4);
+        size_t differ = 0, seen = 0;
+        for (int r = 0; r < m; r += 7)
+            for (int c = 0; c < n; c += 5, seen++) {
+                float sum = 0.0f;
+                for (int b0 = 0; b0 < KB; b0 += kbs) {
+                    float acc = 0.0f;
+                    for (int b = b0; b < KB && b < b0 + kbs; b++) {
+                        const or_block_q8_0 &A = a[(size_t)r * KB + b], &B = w[(size_t)c * KB + b];
+                        int isum = 0;
+                        for (int i = 0; i < 32; i++) isum += A.qs[i] * B.qs[i];
+                        acc = std::fma((float)isum, or_f16_to_f32(A.d) * or_f16_to_f32(B.d), acc);
+                    }
+                    sum += acc;
+                }
+                differ += memcmp(&sum, &got[(size_t)r * n + c], 4) != 0;
+            }
+        printf("split bits %zu of %zu differ, splits %llu tile128 %llu\n", differ, seen, (unsigned long long)gc[3],
+               (unsigned long long)gc[2]);
+        return 0;
+    }
     if (argc == 3 && std::string(argv[1]) == "--step-setup") {
         // a context with the persistent step is set up (SQEMU_STEP=1)
         sq_model* m = nullptr;

@@ -123,6 +123,23 @@ def test_device_token_id_past_the_table_is_an_error(emu):
     assert got == [("3", "63", "0", "0"), ("3", "64", "0", "22"), ("4294967295", "1", "2", "22")], p.stdout
 
 
+@pytest.mark.parametrize("cus,m,n,kbs", [
+    (8, 140, 512, 24),    # 8 tiles of 128 x 128 on 8 CUs: three parts of 24, 24 and 16 blocks
+    (8, 140, 768, 32),    # 12 tiles: two parts
+    (32, 70, 128, 4),     # 4 tiles of 64 x 64 on 32 CUs: 16 parts of one group of four
+])
+def test_k_split_partition(emu, cus, m, n, kbs):
+    """The parts a K split takes, to the last bit of the sums: whole groups of
+    four blocks, on 128 x 128 tiles (what a 2048-token prompt's o and down
+    projections take) as on 64 x 64."""
+    p = subprocess.run([emu, "--split-bits", str(m), "2048", str(n), str(kbs), "5"], capture_output=True, text=True,
+                       env={**ENV, "SQEMU_CUS": str(cus)})
+    assert p.returncode == 0 and "AddressSanitizer" not in p.stderr, p.stdout + p.stderr[-2000:]
+    g = re.search(r"^split bits (\d+) of (\d+) differ, splits (\d+) tile128 (\d)$", p.stdout, re.M)
+    assert g and g[1] == "0" and int(g[2]) > 200, p.stdout
+    assert int(g[3]) == -(-64 // kbs) and g[4] == ("0" if m == 70 else "1"), p.stdout
+
+
 def test_step_setup_waits_for_its_tables(emu, models):
     """The weight-stream builder runs on the context's own stream, which the
     null stream's copies do not order: the layer table it reads has to have
