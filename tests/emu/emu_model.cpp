@@ -105,8 +105,8 @@ int main(int argc, char** argv) {
     }
     if (argc == 2 && std::string(argv[1]) == "--noalloc-count") {
         // hipMalloc calls made by warm calls of sq_linear_noalloc on its two
-        // paths (m = 1: the matvec; m = 67: the K-split matmul), next to
-        // sq_linear's for the same calls
+        // paths (m = 1: the matvec; m = 67: the K-split matmul), next to a
+        // sq_malloc's and those of sq_linear with its scratch given back
         const int k = 2048, n = 256;
         std::vector<uint8_t> w((size_t)n * (k / 32) * 34);
         for (size_t i = 0; i < w.size(); i++) w[i] = (uint8_t)(i * 131 + 7);
@@ -127,10 +127,15 @@ int main(int argc, char** argv) {
             const uint64_t a0 = sqemu::g_malloc_calls;
             if ((st = sq_linear_noalloc(dx, m, k, W, dy, 0))) die("sq_linear_noalloc", st);
             const uint64_t a1 = sqemu::g_malloc_calls;
-            if ((st = sq_linear(dx, m, k, W, dy, 0))) die("sq_linear", st);
+            void* p = nullptr;
+            if ((st = sq_malloc(&p, 64))) die("sq_malloc", st);
+            sq_free(p);
             const uint64_t a2 = sqemu::g_malloc_calls;
-            printf("m %d noalloc_mallocs %llu linear_mallocs %llu\n", m, (unsigned long long)(a1 - a0),
-                   (unsigned long long)(a2 - a1));
+            sq_scratch_trim();
+            if ((st = sq_linear(dx, m, k, W, dy, 0))) die("sq_linear", st);
+            const uint64_t a3 = sqemu::g_malloc_calls;
+            printf("m %d noalloc_mallocs %llu malloc_mallocs %llu linear_mallocs %llu\n", m, (unsigned long long)(a1 - a0),
+                   (unsigned long long)(a2 - a1), (unsigned long long)(a3 - a2));
         }
         return 0;
     }
