@@ -283,12 +283,13 @@ int sq_ctx_time_kernel(sq_ctx* c, int which, int iters, double* mean_us, uint64_
 int sq_ctx_prefill_phases(sq_ctx* c, const uint32_t* ids, size_t n, double* ms);
 /* Matrix-core matmul launches in this process since the last reset
  * (measurement and test aid, no reference counterpart): out[0] all, [1] those
- * that split K over workgroups, [2] those on the full-rate kernel's 128 x 128
- * tiles, [3] the largest split count, [4] those on the full-rate kernel's
- * 128 x 64 tiles, [5] those on the few-rows kernel (32 x 32 tiles, inputs of
- * at most 32 rows) (out holds 6 values).  out may be null; reset != 0 zeroes
- * the counters afterwards. */
+ * that split K over workgroups, [2] those on the tile kernel's 128 x 128
+ * tiles, [3] the largest split count, [4] those on its 128 x 64 tiles, [5] those
+ * on the few-rows kernel (32 x 32 tiles, inputs of at most 32 rows) (out holds 6
+ * values).  out may be null; reset != 0 zeroes the counters afterwards.
+ * _tile64x128_launches: those on 64 x 128 tiles since the same reset. */
 int sq_gemm_counters(int reset, uint64_t* out);
+int sq_gemm_tile64x128_launches(uint64_t* n);
 
 #ifdef __cplusplus
 }

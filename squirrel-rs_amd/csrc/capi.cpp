@@ -200,6 +200,12 @@ int sq_gemm_counters(int reset, uint64_t* out) {
     return 0;
 }
 
+int sq_gemm_tile64x128_launches(uint64_t* n) {
+    if (!n) return set_error(SQ_ERR_ARG, "gemm_tile64x128_launches: null argument");
+    *n = gemm_tile64x128_launches();
+    return 0;
+}
+
 int sq_ctx_act_taps(sq_ctx* c, int enable) {
     if (!c) return set_error(SQ_ERR_ARG, "act_taps: null context");
     return ctx_set_taps(c, enable != 0);

@@ -780,30 +780,24 @@ int device_cus() {
     return cus[dev];
 }
 
-// Matmul launches since the last reset (measurement aid): all, K-split,
-// full-rate 128 x 128 tiles, the largest split count, full-rate 128 x 64
-// tiles.
-std::atomic<uint64_t> g_launches{0}, g_split_launches{0}, g_tile128_launches{0}, g_max_splits{0},
-    g_tile128x64_launches{0}, g_rows_launches{0};
-// bn: 0 for the 64 x 64 kernel, 32 for the few-rows kernel, else the
-// full-rate kernel's tile columns (64 or 128)
-void count_launch(int splits, int bn) {
+// The tile shapes: 128 x 128 outputs a workgroup (four wavefronts of 64 x 64),
+// 128 x 64 (four of 32 x 64), 64 x 64 (two of 32 x 64) and 64 x 128 (four).
+// All fold the same per-block terms in the same order.
+enum : int { SHAPE_128, SHAPE_128X64, SHAPE_64, SHAPE_64X128, SHAPE_ROWS };  // (the last: the few-rows kernel)
+int shape_rows(int shape) { return shape == SHAPE_128 || shape == SHAPE_128X64 ? 128 : 64; }
+int shape_cols(int shape) { return shape == SHAPE_128 || shape == SHAPE_64X128 ? 128 : 64; }
+
+// Matmul launches since the last reset (measurement aid): all, K-split, the
+// largest split count, and by shape.
+std::atomic<uint64_t> g_launches{0}, g_split_launches{0}, g_max_splits{0}, g_shape_launches[SHAPE_ROWS + 1]{};
+void count_launch(int splits, int shape) {
     g_launches++;
-    if (bn == 32) g_rows_launches++;
+    g_shape_launches[shape]++;
     if (splits > 1) g_split_launches++;
-    if (bn == 128) g_tile128_launches++;
-    if (bn == 64) g_tile128x64_launches++;
     uint64_t prev = g_max_splits.load();
     while ((uint64_t)splits > prev && !g_max_splits.compare_exchange_weak(prev, (uint64_t)splits)) {
     }
 }
-
-// The tile shapes: 128 x 128 outputs a workgroup (four wavefronts of 64 x 64),
-// 128 x 64 (four of 32 x 64), 64 x 64 (two of 32 x 64) and 64 x 128 (four).
-// All fold the same per-block terms in the same order.
-enum : int { SHAPE_128 = 128, SHAPE_128X64 = 64, SHAPE_64 = 0, SHAPE_64X128 = 1 };
-int shape_rows(int shape) { return shape == SHAPE_128 || shape == SHAPE_128X64 ? 128 : 64; }
-int shape_cols(int shape) { return shape == SHAPE_128 || shape == SHAPE_64X128 ? 128 : 64; }
 
 FragMat frag(const DevMatrix& w) { return FragMat{(const int8_t*)w.fq, w.fs, w.rows, w.k}; }
 
@@ -846,7 +840,7 @@ int run_tiles(hipStream_t s, int shape, const DevMatrix& w, const int8_t* aq, co
               int ldo, bool acc, int splits, float* ws, const NormThen** then) {
     int kbs;
     k_partition(w.k / 32, &splits, &kbs);
-    count_launch(splits, shape == SHAPE_128 || shape == SHAPE_128X64 ? shape : 0);
+    count_launch(splits, shape);
     if (splits == 1) return launch_shape<WT, RW_STORE>(s, shape, w, aq, ad, m, out, ldo, acc, 1, kbs, 0);
     const size_t stride = (size_t)m * w.rows;
     if (const int st = launch_shape<WT, RW_STORE>(s, shape, w, aq, ad, m, ws, w.rows, false, splits, kbs, stride)) return st;
@@ -923,7 +917,7 @@ int run_rows_shared(hipStream_t s, const DevMatrix* const* ws, int n, const int8
             more.begin[i - 1] = gx;
         }
         gx += (ws[i]->rows + 31) / 32;
-        count_launch(1, 32);
+        count_launch(1, SHAPE_ROWS);
     }
     for (int i = n - 1; i < kSharedMax - 1; i++) more.begin[i] = gx;  // (past the grid)
     const int KB = ws[0]->k / 32;
@@ -942,20 +936,21 @@ int run_rows(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint16_t
     const bool two = p.two;
     const int KB = w.k / 32, gx = p.gx, gy = p.gy, splits = p.splits;
     const int kbs = KB / splits;
-    count_launch(splits, 32);
+    count_launch(splits, SHAPE_ROWS);
     return two ? launch_rows<WT, 2>(s, w, aq, ad, m, out, ldo, acc, gx, gy, splits, kbs, ws, RowsEpi{}, then)
                : launch_rows<WT, 1>(s, w, aq, ad, m, out, ldo, acc, gx, gy, splits, kbs, ws, RowsEpi{}, then);
 }
 
 // SQUIRREL_GEMM_TILE pins the prefill matmul's kernel (a test and
-// measurement aid): "64", "128x64" and "128" the tile kernel on 64 x 64,
-// 128 x 64 or 128 x 128 tiles, "rows" the few-rows kernel.  Unset, inputs of at
+// measurement aid): "64", "64x128", "128x64" and "128" the tile kernel on 64 x 64,
+// 64 x 128, 128 x 64 or 128 x 128 tiles, "rows" the few-rows kernel.  Unset, inputs of at
 // most 32 rows take the few-rows kernel, and larger ones auto_tiling's shape.
-enum : int { TILE_AUTO = 0, TILE_64 = 1, TILE_128X64 = 2, TILE_128 = 3, TILE_ROWS = 4 };
+enum : int { TILE_AUTO, TILE_64, TILE_64X128, TILE_128X64, TILE_128, TILE_ROWS };
 int gemm_tile_override() {
     const char* e = getenv("SQUIRREL_GEMM_TILE");
     if (!e) return TILE_AUTO;
     if (!strcmp(e, "64")) return TILE_64;
+    if (!strcmp(e, "64x128")) return TILE_64X128;
     if (!strcmp(e, "128x64")) return TILE_128X64;
     if (!strcmp(e, "128")) return TILE_128;
     if (!strcmp(e, "rows")) return TILE_ROWS;
@@ -1010,7 +1005,10 @@ int run_integer(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint1
     Tiling t = auto_tiling(w, m, ws, ws_floats);
     if (tile != TILE_AUTO && tile != TILE_ROWS) {
         // pinned: K split below two (64 x 64 tiles: one) workgroups per CU
-        const int cus = device_cus(), shape = tile == TILE_128 ? SHAPE_128 : tile == TILE_128X64 ? SHAPE_128X64 : SHAPE_64;
+        const int cus = device_cus(), shape = tile == TILE_128     ? SHAPE_128
+                                              : tile == TILE_128X64 ? SHAPE_128X64
+                                              : tile == TILE_64X128 ? SHAPE_64X128
+                                                                    : SHAPE_64;
         const int g = (w.rows + shape_cols(shape) - 1) / shape_cols(shape) *
                       ((m + shape_rows(shape) - 1) / shape_rows(shape));
         t = Tiling{shape, shape == SHAPE_64 && g >= cus ? 1 : splits_for(w, m, g, 2 * cus, ws, ws_floats)};
@@ -1063,12 +1061,12 @@ int run_gateup_silu(hipStream_t s, const DevMatrix& w, const int8_t* aq, const u
         if (gemm_tile_override() != TILE_AUTO) return -1;
         const Tiling t = auto_tiling(w, m, ws, ws_floats);
         if (t.splits != 1) return -1;
-        count_launch(1, t.shape == SHAPE_128 || t.shape == SHAPE_128X64 ? t.shape : 0);
+        count_launch(1, t.shape);
         return launch_shape<WT, RW_GATEUP>(s, t.shape, w, aq, ad, m, nullptr, 0, false, 1, (KB + 1) & ~1, 0, ep);
     }
     const int gx = ffn / 32, gy = (m + 31) / 32;
     if (gx * gy < device_cus()) return -1;  // the split-free two-tile form only
-    count_launch(1, 32);
+    count_launch(1, SHAPE_ROWS);
     return launch_rows<WT, 2, RW_GATEUP>(s, w, aq, ad, m, nullptr, 0, false, gx, gy, 1, KB, nullptr, ep);
 }
 
@@ -1089,7 +1087,7 @@ int run_qkv_rope(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint
         k_partition(KB, &t.splits, &kbs);
         // (four columns per thread of the summing kernel)
         if (t.splits > 1 && (ep.q_dim % 4 || ep.kv_dim % 4 || ep.head_dim % 4)) return -1;
-        count_launch(t.splits, t.shape == SHAPE_128 || t.shape == SHAPE_128X64 ? t.shape : 0);
+        count_launch(t.splits, t.shape);
         if (t.splits == 1)
             return launch_shape<WT, RW_QKV>(s, t.shape, w, aq, ad, m, nullptr, 0, false, 1, kbs, 0, ep);
         const size_t stride = (size_t)m * w.rows;
@@ -1103,7 +1101,7 @@ int run_qkv_rope(hipStream_t s, const DevMatrix& w, const int8_t* aq, const uint
     }
     // where run_rows would pair tiles or split K (other sums than the plain path's)
     if ((gx + 1) / 2 * gy >= device_cus() || (gx * gy < device_cus() && KB / (RW_NW * 2 * RW_NB) >= 2)) return -1;
-    count_launch(1, 32);
+    count_launch(1, SHAPE_ROWS);
     return launch_rows<WT, 1, RW_QKV>(s, w, aq, ad, m, nullptr, 0, false, gx, gy, 1, KB, nullptr, ep);
 }
 
@@ -1130,20 +1128,20 @@ void gemm_counters(bool reset, uint64_t* out) {
     if (out) {
         out[0] = g_launches.load();
         out[1] = g_split_launches.load();
-        out[2] = g_tile128_launches.load();
+        out[2] = g_shape_launches[SHAPE_128].load();
         out[3] = g_max_splits.load();
-        out[4] = g_tile128x64_launches.load();
-        out[5] = g_rows_launches.load();
+        out[4] = g_shape_launches[SHAPE_128X64].load();
+        out[5] = g_shape_launches[SHAPE_ROWS].load();
     }
     if (reset) {
         g_launches = 0;
         g_split_launches = 0;
-        g_tile128_launches = 0;
         g_max_splits = 0;
-        g_tile128x64_launches = 0;
-        g_rows_launches = 0;
+        for (auto& n : g_shape_launches) n = 0;
     }
 }
+
+uint64_t gemm_tile64x128_launches() { return g_shape_launches[SHAPE_64X128].load(); }
 
 int launch_gemm_shared(hipStream_t s, const DevMatrix* const* ws, int n, const int8_t* aq, const uint16_t* ad, int m,
                        float* const* outs) {

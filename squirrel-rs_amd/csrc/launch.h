@@ -183,7 +183,9 @@ constexpr size_t kGemmSplitFloats = (size_t)4 << 20;
 constexpr size_t kPrefillSplitFloats = (size_t)16 << 20;
 // Integer matmul launches on the matrix cores since the last reset: out[0]
 // all, [1] with a K split, [2] on 128 x 128 tiles, [3] the largest split.
+// [4] on 128 x 64 tiles, [5] on the few-rows kernel.
 void gemm_counters(bool reset, uint64_t* out);
+uint64_t gemm_tile64x128_launches();
 int launch_gemm(hipStream_t s, const DevMatrix& w, bool a8, const int8_t* aq, const uint16_t* ad,
                 const float* x, int m, float* out, int ldo, bool accumulate,
                 float* ws = nullptr, size_t ws_floats = 0, const NormThen* then = nullptr);

@@ -181,6 +181,13 @@ def gemm_counters(reset: bool = False) -> dict:
             "max_splits": int(out[3]), "tile128x64_launches": int(out[4]), "rows_launches": int(out[5])}
 
 
+def gemm_tile64x128_launches() -> int:
+    """Those launches on 64 x 128 tiles (sq_gemm_tile64x128_launches)."""
+    n = C.c_uint64()
+    check(lib().sq_gemm_tile64x128_launches(C.byref(n)))
+    return n.value
+
+
 def scratch_trim() -> None:
     """Frees the operator calls' idle scratch on the current device (up to
     256 MB), for an allocator of the process that needs the room."""

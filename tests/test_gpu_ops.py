@@ -156,56 +156,83 @@ def test_linear_matches_oracle(wtype, k, n, m, f32_acts):
 
 
 @pytest.mark.parametrize("k", [2048, 8192])
-@pytest.mark.parametrize("tile", ["128x64", "128"])
-def test_direct_to_lds_matmul_matches_register_staged(tile, k, monkeypatch):
+@pytest.mark.parametrize("tile", ["64x128", "128x64", "128"])
+def test_matmul_ragged_tiles_match_oracle(tile, k, monkeypatch):
     """Q8_0 weights on ragged tiles (1000 prompt rows: 7 full 128-row tiles
-    and 104 rows; 4000 columns: 31 full 128-column tiles and 32): the
-    direct-to-LDS kernel (three LDS stages, swizzled rows, loads issued from
-    assembly) and the register-staged kernel (SQUIRREL_GEMM_DMA=0) fold the
-    same per-block terms in the same order, so they agree bit for bit."""
+    and 104 rows; 4000 columns: 31 full 128-column tiles and 32): rows of the
+    first, the inner and the last tile, every column, within 4e-6 of the sum
+    of |terms| of the oracle (matmul.rs:133-171), and all of it bit for bit
+    what 64 x 64 tiles give (the same terms in the same order)."""
     m, n = 1000, 4000
     w, _ = quant_weights(O.Q8_0, n, k, seed=91)
     x = (rng(5).standard_normal((m, k)) * 1.5).astype(np.float32)
     W = ops.Weight(O.Q8_0, w, n, k)
     d_x = DeviceArray.from_numpy(x)
-    monkeypatch.setenv("SQUIRREL_GEMM_TILE", tile)
     outs = {}
-    for dma in ("1", "0"):
-        monkeypatch.setenv("SQUIRREL_GEMM_DMA", dma)
+    for t in (tile, "64"):
+        monkeypatch.setenv("SQUIRREL_GEMM_TILE", t)
         out = DeviceArray((m, n))
         ops.gemm_counters(reset=True)
         ops.linear(d_x, W, out)
+        wide = ops.gemm_tile64x128_launches()
         got = ops.gemm_counters(reset=True)
         assert got["launches"] == 1 and got["split_launches"] == 0, got
-        outs[dma] = out.numpy()
-    assert np.array_equal(outs["1"], outs["0"])
-    assert np.all(np.isfinite(outs["1"]))
+        assert (got["tile128_launches"], got["tile128x64_launches"], wide) == (t == "128", t == "128x64", t == "64x128")
+        outs[t] = out.numpy()
+    rows = np.array([0, 31, 32, 127, 128, 500, 895, 896, 959, 960, 991, 992, 999])
+    want = O.linear(x[rows], O.Q8_0, w, n, O.W8A8)
+    wf = np.stack([O.dequantize(O.Q8_0, w[i], k) for i in range(n)])
+    assert np.all(np.abs(outs[tile][rows].astype(np.float64) - want) <= 4e-6 * term_mag(x[rows], wf) + 1e-6)
+    assert np.array_equal(outs[tile], outs["64"])
+
+
+@pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("m,k,n", [(131, 2080, 16416), (300, 160, 10000)])
+def test_matmul_wide_ragged_input_takes_64_row_tiles(wtype, m, k, n):
+    """Matrices of 8192 and more rows and an input whose last 128-row tile
+    would be mostly empty take 64 x 128 tiles with no tiling pinned: last tiles
+    of 32 and 16 columns, of 3 and 44 rows, and odd counts of blocks (65, 5),
+    against the oracle as above."""
+    w, _ = quant_weights(wtype, n, k, seed=5 + m)
+    x = (rng(m).standard_normal((m, k)) * 1.5).astype(np.float32)
+    out = DeviceArray((m, n))
+    ops.gemm_counters(reset=True)
+    ops.linear(DeviceArray.from_numpy(x), ops.Weight(wtype, w, n, k), out)
+    wide = ops.gemm_tile64x128_launches()
+    c = ops.gemm_counters(reset=True)
+    assert c["launches"] == 1 and c["split_launches"] == 0 and wide == 1, (c, wide)
+    rows = np.array(sorted({0, 31, 32, 63, 64, 127, 128, m - 1}))
+    want = O.linear(x[rows], wtype, w, n, O.W8A8)
+    wf = np.stack([O.dequantize(wtype, w[i], k) for i in range(n)])
+    assert np.all(np.abs(out.numpy()[rows].astype(np.float64) - want) <= 4e-6 * term_mag(x[rows], wf) + 1e-6)
 
 
 @pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0])
 def test_matmul_tiles_agree(wtype, monkeypatch):
-    """The prefill matmul's three tilings (64 x 64 on v_mfma_i32_16x16x32_i8,
-    128 x 64 and 128 x 128 on v_mfma_i32_32x32x32_i8) fold the same per-block
-    terms in the same order for every output, so without a K split they agree
-    bit for bit; the 128 x 128 result also matches the oracle
+    """The prefill matmul's four tile shapes (64 x 64, 64 x 128, 128 x 64 and
+    128 x 128, wavefronts of one to four 32 x 32 tiles) fold the same
+    per-block terms in the same order for every output, so without a K split
+    they agree bit for bit; the 128 x 128 result also matches the oracle
     (matmul.rs:133-171)."""
-    m, k, n = 1024, 2048, 4096      # 1024, 512 and 256 tiles: no kernel splits K
+    m, k, n = 1024, 2048, 4096      # 1024, 512, 512 and 256 tiles: no shape splits K
     w, _ = quant_weights(wtype, n, k, seed=77 + wtype)
     x = (rng(3).standard_normal((m, k)) * 1.5).astype(np.float32)
     W = ops.Weight(wtype, w, n, k)
     d_x = DeviceArray.from_numpy(x)
     outs = {}
-    for tile in ("64", "128x64", "128"):
+    for tile in ("64", "64x128", "128x64", "128"):
         monkeypatch.setenv("SQUIRREL_GEMM_TILE", tile)
         out = DeviceArray((m, n))
         ops.gemm_counters(reset=True)
         ops.linear(d_x, W, out)
+        assert ops.gemm_tile64x128_launches() == (1 if tile == "64x128" else 0)
         got = ops.gemm_counters(reset=True)
         assert got["launches"] == 1 and got["split_launches"] == 0, got
         assert got["tile128_launches"] == (1 if tile == "128" else 0), got
         assert got["tile128x64_launches"] == (1 if tile == "128x64" else 0), got
         outs[tile] = out.numpy()
     assert np.array_equal(outs["64"], outs["128"])
+    assert np.array_equal(outs["64x128"], outs["128"])
     assert np.array_equal(outs["128x64"], outs["128"])
     rows = np.arange(0, m, 97)
     want = O.linear(x[rows], wtype, w, n, O.W8A8)
@@ -249,7 +276,7 @@ def test_matmul_rows_kernel_matches_oracle(wtype, m, k, n, pin, monkeypatch):
 
 
 @pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0])
-@pytest.mark.parametrize("pin", [None, "64", "128x64", "128"])
+@pytest.mark.parametrize("pin", [None, "64", "64x128", "128x64", "128"])
 @pytest.mark.parametrize("m,k,n", [
     (33, 32, 1), (63, 96, 33), (65, 160, 100), (97, 224, 129), (128, 64, 64), (131, 2048, 300), (257, 288, 65),
     (2, 4128, 40),
@@ -265,7 +292,9 @@ def test_matmul_fragment_order_edges(wtype, pin, m, k, n, monkeypatch):
     w, _ = quant_weights(wtype, n, k, seed=7 + m)
     x = (rng(m + k).standard_normal((m, k)) * 1.5).astype(np.float32)
     out = DeviceArray((m, n))
+    ops.gemm_counters(reset=True)
     ops.linear(DeviceArray.from_numpy(x), ops.Weight(wtype, w, n, k), out)
+    assert ops.gemm_tile64x128_launches() == (1 if pin == "64x128" else 0)
     got = out.numpy().astype(np.float64)
     want = O.linear(x, wtype, w, n, O.W8A8)
     wf = np.stack([O.dequantize(wtype, w[i], k) for i in range(n)])
@@ -494,9 +523,9 @@ def test_sdpa_model_kernels_match_oracle(seq_q, seq_k, nh, nkv, attn, monkeypatc
 @pytest.mark.parametrize("nh,nkv", [(32, 8), (4, 2), (8, 1), (3, 3)])
 def test_sdpa_decode_tile_edges(seq_k, nh, nkv):
     """One query over key counts around the 64-position tiles, the merge's 64
-    tiles per round and its 16 loads in flight, for every GQA group size;
-    an infinite V row past the keys (the same buffer's next row) is not read
-    into the result.  The bound of the test above: outputs are convex
+    tiles per round and its 16 loads in flight, for every GQA group size; the
+    rows past the keys (the same buffers' next tile, infinite and NaN) do not
+    reach the result.  The bound of the test above: outputs are convex
     combinations of v rows."""
     hd = 64
     r = rng(seq_k + nh)
@@ -505,8 +534,17 @@ def test_sdpa_decode_tile_edges(seq_k, nh, nkv):
     v = r.standard_normal(seq_k * nkv * hd).astype(np.float32)
     st, want = O.sdpa(q, k, v, 1, seq_k, nh, nkv, hd)
     assert st == 0
-    got = sdpa_dev(q, k, v, 1, seq_k, nh, nkv, hd)
-    assert np.allclose(got, want, rtol=1e-5, atol=2e-6), float(np.abs(got - want).max())
+
+    class Head:  # the first seq_k rows of a longer buffer
+        def __init__(self, rows, past):
+            self.buf = DeviceArray.from_numpy(np.concatenate([rows, np.full(64 * nkv * hd, past, np.float32)]))
+            self.ptr, self.size = self.buf.ptr, rows.size
+
+    for past_k, past_v in ((np.inf, np.inf), (np.nan, np.nan)):
+        out = DeviceArray(q.size)
+        ops.sdpa_cached(DeviceArray.from_numpy(q), Head(k, past_k), Head(v, past_v), out, nh, nkv, hd)
+        got = out.numpy()
+        assert np.allclose(got, want, rtol=1e-5, atol=2e-6), float(np.abs(got - want).max())
     # an infinite last row reaches the output as infinities, not NaN
     v[-nkv * hd:] = np.inf
     got = sdpa_dev(q, k, v, 1, seq_k, nh, nkv, hd)
