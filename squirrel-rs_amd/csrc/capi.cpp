@@ -155,7 +155,8 @@ int sq_ctx_step_trace(sq_ctx* c, int enable) {
     }
     const int stride = 20 * c->m->cfg.n_layers + 4;
     if (!c->s_trace) SQ_HIP_CHECK(device_alloc((void**)&c->s_trace, (size_t)c->step_grid * stride * 8));
-    SQ_HIP_CHECK(hipMemset(c->s_trace, 0, (size_t)c->step_grid * stride * 8));
+    // (on the stream of the steps that write it)
+    SQ_HIP_CHECK(hipMemsetAsync(c->s_trace, 0, (size_t)c->step_grid * stride * 8, c->stream));
     c->step.trace = c->s_trace;
     c->step.trace_stride = stride;
     return 0;

@@ -267,6 +267,15 @@ int main(int argc, char** argv) {
         sq_ctx* c = nullptr;
         if ((st = sq_ctx_new(m, 64, 0, &c))) die("sq_ctx_new", st);
         printf("step set up %d\n", sq_ctx_decode_kernel(c));
+        // its timeline is cleared before the next step, not after it
+        const uint32_t id = 3;
+        int grid = 0, stride = 0;
+        if ((st = sq_ctx_step_trace(c, 1))) die("sq_ctx_step_trace", st);
+        if ((st = sq_forward(m, c, &id, 1))) die("sq_forward", st);
+        if ((st = sq_ctx_step_trace_read(c, nullptr, 0, &grid, &stride))) die("sq_ctx_step_trace_read", st);
+        std::vector<uint64_t> trace((size_t)grid * stride);
+        if ((st = sq_ctx_step_trace_read(c, trace.data(), trace.size(), &grid, &stride))) die("sq_ctx_step_trace_read", st);
+        printf("step trace %llu %llu\n", (unsigned long long)trace[0], (unsigned long long)trace[1]);
         sq_ctx_free(c);
         sq_model_free(m);
         return 0;

@@ -145,10 +145,12 @@ def test_k_split_partition(emu, cus, m, n, kbs):
 def test_step_setup_waits_for_its_tables(emu, models):
     """The weight-stream builder runs on the context's own stream, which the
     null stream's copies do not order: the layer table it reads has to have
-    arrived."""
+    arrived.  And the step timeline's buffer is cleared on that stream, not
+    behind its steps' backs."""
     p = subprocess.run([emu, "--step-setup", models["Q8_0"]], capture_output=True, text=True,
                        env={**ENV, "SQEMU_STEP": "1"})
     assert p.returncode == 0 and "step set up 1" in p.stdout, p.stdout + p.stderr[-2000:]
+    assert "step trace 7 0" in p.stdout, p.stdout
 
 
 def test_scratch_pool_bounds(emu):
