@@ -55,8 +55,9 @@ MATMUL_ELEMS_PER_LAYER = 60817408
 # One 32x32 output tile and 32-element block of the int8 matmul (65536 ops) with
 # all its operands in registers, per SIMD: the matrix instructions, and the
 # subtraction and the fused multiply-add of each element (the scale product
-# comes from the f16 matrix instruction).  Measured.
-RESCALE_TILE_NS = 47.0
+# comes from the f16 matrix instruction).  Measured on two wavefronts of four
+# tiles a SIMD: 41 in launches of milliseconds, 47 in ones of 0.2 ms.
+RESCALE_TILE_NS = 41.0
 CONFIGS = {
     "q8": dict(wtype="Q8_0", prompt=32, gen=64,
                workload="Llama-3.2-1B arch, Q8_0 GGUF, 32-token prompt then 64 greedy tokens"),

@@ -152,7 +152,9 @@ typedef float m8_v16f __attribute__((ext_vector_type(16)));
 // a block's sum is at most 32 * 127 * 128), and one subtraction leaves
 // f32(isum), exactly.  v_cvt_f32_i32 issues at half the rate of a subtraction
 // (2.4 against 1.3 ns per wavefront instruction and SIMD), and with it a
-// 32 x 32 tile and block took 61 ns per SIMD in registers alone, against 41 ns.
+// 32 x 32 tile and block takes 50 ns per SIMD in registers alone, against 41 ns
+// (two wavefronts of four tiles a SIMD, launches of 2.6 ms; 57 and 47 in
+// launches of 0.2 ms; three wavefronts: 59 and 43).
 // The base operand sits in registers, behind an empty asm so that the compiler
 // does not set it anew for every product.
 constexpr int kIsumBase = 0x4B400000;
@@ -969,11 +971,17 @@ bool rows_kernel_fits(int m, int k) { return m <= 32 && (k / 32) % RW_NB == 0 &&
 //    64 x 64: 156 against 137 us for 2048 x 16384 x 2048; of 320 rows, 384 in
 //    128-row tiles, 37 against 41);
 //  - 128 x 128 tiles where they give every CU two workgroups;
-//  - where 128 x 128 tiles cover a third to a half of the device's
-//    three-per-CU slots, the same tiles with K split two or three ways (one
-//    round; the partials summed in split order): the o and FFN down projections
-//    of a 2048-token prompt (256 tiles) three ways, its q|k|v projection (384
-//    tiles) two;
+//  - where they give one to two (on 256 CUs 256 to 511 tiles, a third to two
+//    thirds of the three-per-CU slots) and the matrix has fewer than 8192 rows,
+//    the same tiles with K split two or three ways, the partials summed in
+//    split order: the o and FFN down projections of a 2048-token prompt (256
+//    tiles) three ways, its q|k|v projection (384 tiles) two, one round each.
+//    Counts that do not divide the slots leave a second round partly empty
+//    (q|k|v of 1800 rows, 360 tiles in three splits: 51 us alone, 46 in two);
+//  (8192 rows stand between the 1B model's gate/up projection, 16384, and its
+//  others, at most 3072; nothing lies between in a model.  On 8160 rows, which
+//  the rule splits, 700 input rows take 47 us and 35 on unsplit 64 x 128 tiles:
+//  the line is not drawn where the two meet)
 //  - 128 x 64 tiles where those give every CU two workgroups;
 //  - else 64 x 64 tiles, and where these are fewer than the CUs, K split over
 //    about two workgroups per CU.
