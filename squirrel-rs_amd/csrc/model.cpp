@@ -224,8 +224,8 @@ int upload_stacked(int wtype, const std::vector<const uint8_t*>& parts, const st
     if (frag) {
         out->fq = (uint8_t*)out->qs + f_off;
         out->fs = (uint16_t*)((uint8_t*)out->fq + up256(q_bytes));
-        // on the null stream, as the operators' launches are; a context's own
-        // stream starts after the device has been waited for
+        // on the null stream, as the operators' launches are (model_load waits
+        // for it)
         if ((st = launch_frag_copy(nullptr, *out))) return st;
     }
     return 0;
@@ -376,6 +376,10 @@ int model_load_impl(const char* path, sq_model** out, bool upload, bool frag) {
     m->tied = tied;
     m->weight_bytes += m->head.payload_bytes() + m->head.scale_bytes();
     m->wtype = wtype;
+    // a context's own stream, which the null stream does not order, reads the
+    // matrices while it is set up
+    if (const hipError_t e = hipStreamSynchronize(nullptr))
+        return fail(set_error(SQ_ERR_HIP, std::string("load: ") + hipGetErrorString(e)));
     *out = m;
     return 0;
 }
@@ -785,7 +789,8 @@ int setup_persistent(sq_ctx* c) {
         (st = dmalloc(&c->s_epoch, 1)))
         return st;
     c->s_error = (int*)(c->d_id_error + 1);
-    SQ_HIP_CHECK(hipMemcpy(c->d_layers, hl.data(), hl.size() * sizeof(StepLayer), hipMemcpyHostToDevice));
+    // on the stream of the kernel that reads it (the null stream does not order it)
+    SQ_HIP_CHECK(hipMemcpyAsync(c->d_layers, hl.data(), hl.size() * sizeof(StepLayer), hipMemcpyHostToDevice, c->stream));
     SQ_HIP_CHECK(hipMemset(c->s_xchg, 0, nx * 8));
     SQ_HIP_CHECK(hipMemset(c->s_epoch, 0, 4));
     SQ_HIP_CHECK(hipMemset(c->s_error, 0, 4));
@@ -839,9 +844,6 @@ int setup_persistent(sq_ctx* c) {
     a.stream_stride = decode_stream_stride(m->wtype, g.n_layers, g.dim, g.ffn, g.n_heads, g.n_kv_heads, g.vocab, grid);
     if ((st = dmalloc(&c->s_stream, a.stream_stride * 16 * (size_t)grid))) return st;
     a.stream = c->s_stream;
-    // the table and the matrices came over the null stream, which does not
-    // order this context's own
-    SQ_HIP_CHECK(hipDeviceSynchronize());
     if ((st = launch_build_stream(c->stream, m->wtype, a, grid, c->s_stream))) return st;
     SQ_HIP_CHECK(hipStreamSynchronize(c->stream));
     c->step_grid = grid;
