@@ -975,8 +975,8 @@ bool rows_kernel_fits(int m, int k) { return m <= 32 && (k / 32) % RW_NB == 0 &&
 //    thirds of the three-per-CU slots) and the matrix has fewer than 8192 rows,
 //    the same tiles with K split two or three ways, the partials summed in
 //    split order: the o and FFN down projections of a 2048-token prompt (256
-//    tiles) three ways, its q|k|v projection (384 tiles) two, one round each.
-//    Counts that do not divide the slots leave a second round partly empty
+//    tiles) three ways, its q|k|v projection (384 tiles) two, every slot
+//    taken once.  Counts that do not divide the slots leave the last ones empty
 //    (q|k|v of 1800 rows, 360 tiles in three splits: 51 us alone, 46 in two);
 //  (8192 rows stand between the 1B model's gate/up projection, 16384, and its
 //  others, at most 3072; nothing lies between in a model.  On 8160 rows, which

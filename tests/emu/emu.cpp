@@ -533,7 +533,7 @@ hipError_t hipDeviceSynchronize() {
 }
 namespace sqemu {
 uint64_t g_malloc_calls = 0;
-size_t g_dev_cap = SIZE_MAX;  // device bytes that hipMalloc may hand out together (a driver sets it)
+size_t g_dev_cap = SIZE_MAX;  // device bytes that hipMalloc may hand out together (a test program sets it)
 size_t dev_bytes() {          // live device bytes
     size_t n = 0;
     for (auto& b : g_dev) n += b.second;
